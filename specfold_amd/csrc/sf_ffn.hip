@@ -287,12 +287,12 @@ constexpr int kFixRows = 8;
 __global__ __launch_bounds__(256) void down_fixup_kernel(const float* __restrict__ part, Plan plan,
                                                          int mcap, const int32_t* __restrict__ rows,
                                                          const int32_t* __restrict__ count_p, int N,
-                                                         uint16_t* __restrict__ out) {
+                                                         uint16_t* __restrict__ out, TilePlans tp) {
   const int t = blockIdx.x;
-  const int first = tile_first(t, plan);
-  const int nsl = tile_last(t, plan) - first + 1;
-  if (nsl == 1) return;
   const int M = min(*count_p, mcap);
+  const int nsl = tile_last(t, plan) - tile_first(t, plan) + 1;
+  // (the tile GEMM leaves single slots to this kernel too)
+  if (nsl == 1 && !(M > kTileRows && tp.nt)) return;
   const int m = blockIdx.y * kFixRows + (threadIdx.x >> 5);
   if (m >= M) return;
   const size_t stride = (size_t)mcap * N;
@@ -375,6 +375,16 @@ Plan gate_up_plan(int I, int S) {
   if (nu >= 2 * SFG_GRID && nu <= 8 * SFG_GRID)
     return make_plan_spread(nu, S, spread_workgroups(nu, SFG_GRID));
   return make_plan(I / 128, S);
+}
+
+// The tile GEMM's shapes for a plan whose K ranges are the same for every column (the
+// spread plan's whole K, a split plan's ranges); none for a stream-K plan, whose cuts
+// differ from tile to tile.
+TilePlans down_tiles(const Plan& p, int N, int K) {
+  return p.KS ? make_tile_plans(N / 16, K, false, p.KS) : TilePlans{};
+}
+TilePlans gate_up_tiles(const Plan& p, int I, int K) {
+  return p.NU ? make_tile_plans(I / 16, K, true, 1) : TilePlans{};
 }
 
 }  // namespace
@@ -518,7 +528,7 @@ extern "C" int sf_ffn_gate_up(const uint16_t* zn, const int32_t* count, int buck
   ep.out = act;
   ep.ldo = I;
   // whole tiles get SiLU*mul straight from registers, shared tiles in the fix-up
-  launch_sk<2, kSilu>(p, zn, nullptr, D, count, 0, bucket, wg, wu, D, I, part, ep, st);
+  launch_sk<2, kSilu>(p, gate_up_tiles(p, I, D), zn, nullptr, D, count, 0, bucket, wg, wu, D, I, part, ep, st);
   if (p.U < p.S)
     hipLaunchKernelGGL(silu_fixup_kernel, dim3(p.T, (bucket + kFixRows - 1) / kFixRows), dim3(256),
                        0, st, part, p, bucket, count, I, act);
@@ -539,9 +549,10 @@ extern "C" int sf_ffn_down_scatter(const uint16_t* act, const int32_t* count, in
   ep.rows = rows;
   ep.out = ffn;
   ep.ldo = D;
-  launch_sk<1, kScatter>(p, act, nullptr, I, count, 0, bucket, wd, nullptr, I, D, part, ep, st);
+  const TilePlans tp = down_tiles(p, D, I);
+  launch_sk<1, kScatter>(p, tp, act, nullptr, I, count, 0, bucket, wd, nullptr, I, D, part, ep, st);
   hipLaunchKernelGGL(down_fixup_kernel, dim3(p.T, (bucket + kFixRows - 1) / kFixRows), dim3(256), 0,
-                     st, part, p, bucket, rows, count, D, ffn);
+                     st, part, p, bucket, rows, count, D, ffn, tp);
   return sf_launch_status();
 }
 

@@ -20,6 +20,7 @@
 #include "sf_common.h"
 #include "sf_compact.h"
 #include "sf_index.h"
+#include "sf_gemm_tile.h"
 
 namespace sfg {
 
@@ -304,18 +305,19 @@ struct GateIn {
 // one pass per MB rows).  Grid: plan_grid workgroups.
 // part: fp32 partial slots [slot][mcap][N] ([slot][mcap][2N] for kSilu).
 // GATED: rows and the count come from the compaction of gate.rec (mcap = bucket).
-template <int WN, int MODE, int MB, bool GATED = false>
+template <int WN, int MODE, int MB, bool GATED = false, bool TILE = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_sk_kernel(const uint16_t* __restrict__ A, const int32_t* __restrict__ a_rows, int lda,
                     const int32_t* __restrict__ count_p, int m_static, int mcap,
                     const uint16_t* __restrict__ W0, const uint16_t* __restrict__ W1, int K, int N,
-                    Plan plan, float* __restrict__ part, Epi ep, GateIn gate) {
+                    Plan plan, float* __restrict__ part, Epi ep, GateIn gate, TilePlans tp) {
   constexpr int kMT = MB / 16;    // max m tiles of this kernel
   using St = Stage<MB, WN>;
   constexpr int R = St::kRing;
   // the ring, whose memory then holds each piece's fp32 tile for the epilogue
   constexpr int kTileWords = TileLds<WN, MB, MODE == kSilu>::kFloats / 4;
-  constexpr int kRingWords = R * St::kWords > kTileWords ? R * St::kWords : kTileWords;
+  constexpr int kStreamWords = R * St::kWords > kTileWords ? R * St::kWords : kTileWords;
+  constexpr int kRingWords = TILE ? kLdsBudget / 16 : kStreamWords;
   __shared__ sf_u32x4 ring[kRingWords];
   __shared__ int rows_s[MB];
   __shared__ int s_grows[GATED ? kGateMaxRows : 1];      // the compacted rows
@@ -331,6 +333,23 @@ void gemm_sk_kernel(const uint16_t* __restrict__ A, const int32_t* __restrict__ 
     M = sf_imin(total, mcap);
   } else {
     M = count_p ? sf_imin(*count_p, mcap) : m_static;
+  }
+  if constexpr (TILE) {
+    // workgroup-uniform: more rows than a pass below holds (and a plan the tile GEMM
+    // computes with the same sums: tp.nt = 0 otherwise)
+    if (M > kTileRows && tp.nt) {
+      const TileGemm tg{A, lda, W0, W1, K, N / 16};
+      auto in_row = [&](int r) { return GATED ? s_grows[r] : (a_rows ? a_rows[r] : r); };
+      if constexpr (MODE == kSilu) {
+        tile_gemm<true>(tg, M, tp, ring, in_row, TileSiluStore{ring, ep.out, ep.ldo, N / 16});
+      } else {
+        // kScatter too: the fix-up scatters every tile
+        static_assert(MODE == kPart || MODE == kScatter, "tile modes");
+        tile_gemm<false>(tg, M, tp, ring, in_row, TilePartStore{part, mcap, N});
+      }
+      return;
+    }
+    if ((int)blockIdx.x >= plan_grid(plan)) return;   // the tile path's workgroups
   }
   Ring<MB, WN> rg;
 #pragma unroll
@@ -462,20 +481,25 @@ void gemm_sk_kernel(const uint16_t* __restrict__ A, const int32_t* __restrict__ 
   }  // row passes
 }
 
-// One pass over the weights for every row: the row block MB is the smallest of
-// 64 / 128 / 256 that holds mcap rows (A ring 8 / 8 / 4 stages, 64 / 128 / 128 KB).
+// The kernel for a launch of at most mcap rows: 64 rows, 128 rows, or 128 rows with
+// the tile GEMM for device-side counts above that (one pass over the weights for
+// every 256 rows, where the streaming core would take one per 128).
 template <int WN, int MODE, bool GATED = false>
-inline void launch_sk(const Plan& p, const uint16_t* A, const int32_t* a_rows, int lda,
-                      const int32_t* count_p, int m_static, int mcap, const uint16_t* W0,
+inline void launch_sk(const Plan& p, const TilePlans& tp, const uint16_t* A, const int32_t* a_rows,
+                      int lda, const int32_t* count_p, int m_static, int mcap, const uint16_t* W0,
                       const uint16_t* W1, int K, int N, float* part, const Epi& ep,
                       hipStream_t st, const GateIn& gate = GateIn{}) {
   const dim3 grid(plan_grid(p));
   if (row_block(mcap) == 64)
     hipLaunchKernelGGL((gemm_sk_kernel<WN, MODE, 64, GATED>), grid, dim3(kThreads), 0, st, A,
-                       a_rows, lda, count_p, m_static, mcap, W0, W1, K, N, p, part, ep, gate);
-  else
+                       a_rows, lda, count_p, m_static, mcap, W0, W1, K, N, p, part, ep, gate, tp);
+  else if (mcap <= kTileRows)
     hipLaunchKernelGGL((gemm_sk_kernel<WN, MODE, 128, GATED>), grid, dim3(kThreads), 0, st, A,
-                       a_rows, lda, count_p, m_static, mcap, W0, W1, K, N, p, part, ep, gate);
+                       a_rows, lda, count_p, m_static, mcap, W0, W1, K, N, p, part, ep, gate, tp);
+  else
+    hipLaunchKernelGGL((gemm_sk_kernel<WN, MODE, 128, GATED, true>), dim3(SFG_GRID),
+                       dim3(kThreads), 0, st, A, a_rows, lda, count_p, m_static, mcap, W0, W1, K,
+                       N, p, part, ep, gate, tp);
 }
 
 }  // namespace sfg

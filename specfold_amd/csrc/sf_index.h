@@ -58,6 +58,16 @@ SF_IDX int a_swz(int r) { return (r >> 1) & 3; }
 SF_IDX int a_copy(int wv, int j, int NMT) { return sf_imin(wv + 8 * j, 2 * NMT - 1); }
 SF_IDX int a_copy_unit(int L) { return (L & 3) ^ a_swz(L >> 2); }
 SF_IDX int a_read_word(int l) { return (l & 15) * 4 + ((l >> 4) ^ a_swz(l & 15)); }
+// The same for a whole 64-K stage at once: 16 rows x 128 bytes, two copies of 8 rows
+// each, so every copy takes whole 128-byte cache lines.  (Two copies that share a
+// line stall the vector cache: the second hits a line whose data is still on its way.)
+// Word r*8 + (u ^ r%8) holds unit u of row r: lane L of a copy brings unit
+// a2_copy_unit(L) of row L/8; the fragment reader lane l of chunk k (unit 4k + l/16 of
+// row l%16) reads word a2_read_word(l, k).
+SF_IDX int a2_copy_unit(int L) { return (L & 7) ^ (L >> 3); }
+SF_IDX int a2_read_word(int l, int k) {
+  return (l & 15) * 8 + ((4 * k + (l >> 4)) ^ (l & 7));
+}
 
 // Output column held by lane `lane` of wave `wv` (its column group) in its column
 // tile `tt` of 128·WN-column tile t (WN tiles of 16 per wave).  SILU: the gate and
@@ -111,15 +121,15 @@ SF_IDX int spread_workgroups(int nu, int grid) {
 // each hold a single piece -- no range crosses a tile, so no workgroup pays a
 // second ring fill and epilogue (the stream-K ranges that straddle two tiles
 // finish last) -- and range j of a tile goes to partial slot j.  KS is the most
-// that keeps T·KS within the grid.
-inline Plan make_plan_split(int T, int S) {
+// that keeps T·KS within the grid and min_stages stages in a range.
+inline Plan make_plan_split(int T, int S, int min_stages = 1) {
   int ks = SFG_GRID / T;
-  ks = ks < 1 ? 1 : (ks > S ? S : ks);
+  ks = sf_imax(1, sf_imin(ks, S / min_stages));
   return Plan{T, S, (S + ks - 1) / ks, 0, ks};
 }
 SF_IDX int split_begin(int j, const Plan& p) { return (int)((long long)j * p.S / p.KS); }
 
-inline int plan_grid(const Plan& p) {
+SF_IDX int plan_grid(const Plan& p) {
   if (p.KS) return p.T * p.KS;
   return (int)(((long long)p.T * p.S + p.U - 1) / p.U);
 }
@@ -254,6 +264,59 @@ SF_IDX int rows_w_chunk(int q, int CPS) { return q % CPS; }
 // fp32 partials of a plan for M rows and N columns: [KS][M][N].
 inline size_t rows_part_bytes(const RowsPlan& p, int M, int N) {
   return p.KS > 1 ? (size_t)p.KS * M * N * sizeof(float) : 0;
+}
+
+// ---------------------------------------------------------------------------
+// Tile GEMM (sf_gemm_tile.h): more than kTileRows rows.  M rows are cut into
+// tile_blocks(M) blocks of at most 256, all of 64·tile_nmt(M) rows (the last one
+// shorter); a workgroup tile is one block by 32·NT columns, K cut into ks ranges.
+constexpr int kTileRows = 128;       // rows one pass of the streaming core holds
+constexpr int kTileMaxBlocks = 4;    // <= 1024 rows
+SF_IDX int tile_blocks(int M) { return (M + 255) / 256; }
+SF_IDX int tile_nmt(int M) {
+  const int nb = tile_blocks(M);
+  return (M + nb - 1) / nb <= 192 ? 3 : 4;
+}
+struct TilePlans {
+  int ks = 1;        // K ranges
+  unsigned nt = 0;   // byte tile_blocks(M) - 1: NT
+};
+SF_IDX int tile_nt(int M, const TilePlans& p) { return (p.nt >> (8 * (tile_blocks(M) - 1))) & 255; }
+// Cycles of a workgroup per 32-wide K chunk: the LDS operand reads of 8 waves
+// (128 B a cycle) with the copies' writes, or two waves' MFMAs per SIMD.
+inline long long tile_chunk_cycles(int nmt, int nt) {
+  const long long lds = (nmt + nt) * 64 + (4 * nmt + 2 * nt) * 8;
+  const long long mfma = nmt * nt * 32;
+  return lds > mfma ? lds : mfma;
+}
+// NT of the tile GEMM of `units` 16-column units (silu: gate units; the up units are
+// as many again) over K in ks ranges, for every row-block count: the lowest estimate
+// of whole rounds of the grid (never below the weight stream, ~2000 bytes a cycle)
+// and a fixed cost per item.  The K ranges are those of the streaming core's plan
+// (a whole K, or its split plan), so a row's sums are the same for every row count.
+inline TilePlans make_tile_plans(int units, int K, bool silu, int ks) {
+  TilePlans p;
+  p.ks = ks;
+  for (int b = 1; b <= kTileMaxBlocks; ++b) {
+    long long best = -1;
+    unsigned best_nt = 0;
+    for (int nt = 2; nt <= 8; ++nt) {
+      if (silu ? nt == 2 : (nt != 2 && nt != 4 && nt != 8)) continue;
+      const int per = silu ? nt : 2 * nt;
+      const int T = (units + per - 1) / per;
+      const long long rounds = ((long long)T * b * ks + SFG_GRID - 1) / SFG_GRID;
+      long long cost = rounds * ((K / 32 + ks - 1) / ks) * tile_chunk_cycles(4, nt);
+      const long long stream = (long long)units * (silu ? 2 : 1) * K * 32 / 2000;
+      if (cost < stream) cost = stream;
+      cost += rounds * 6000;
+      if (best < 0 || cost < best) {
+        best = cost;
+        best_nt = (unsigned)nt;
+      }
+    }
+    p.nt |= best_nt << (8 * (b - 1));
+  }
+  return p;
 }
 
 }  // namespace sfg

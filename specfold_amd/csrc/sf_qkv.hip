@@ -34,11 +34,11 @@ __global__ __launch_bounds__(256) void sf_qkv_epilogue_kernel(
   const int t = threadIdx.x & 63;
   const int c0 = head * 128 + t;
   const int c1 = c0 + 64;
-  const int nsl = tile_last(head, plan) - tile_first(head, plan) + 1;
   const size_t stride = (size_t)bucket * n_qkv;
   const float b0 = bias ? sf_bf2f(bias[c0]) : 0.f;
   const float b1 = bias ? sf_bf2f(bias[c1]) : 0.f;
   const int count = min(*count_p, bucket);
+  const int nsl = tile_last(head, plan) - tile_first(head, plan) + 1;
   const int p0 = (!BRANCHES && pos0) ? *pos0 : 0;
   for (int m = blockIdx.x; m < count; m += gridDim.x) {
     const int row = rows[m];
@@ -80,11 +80,27 @@ __global__ __launch_bounds__(256) void sf_qkv_epilogue_kernel(
   }
 }
 
+// Each head's tile cut into whole K ranges (split plan, as FFN down) while the heads
+// are fewer than the grid: the same ranges for every head, so that the tile GEMM (more
+// than 128 rows) gives every row the streaming core's sums.  A range holds at least
+// three 64-K stages: shorter ones are all ring fill, and their partial slots cost the
+// epilogue more than the idle CUs do the GEMM.
+Plan qkv_plan(int n_qkv, int D) {
+  const int T = n_qkv / 128, S = D / kKC;
+  return T < SFG_GRID ? make_plan_split(T, S, 3) : make_plan(T, S);
+}
+TilePlans qkv_tiles(const Plan& p, int n_qkv, int D) {
+  return p.KS ? make_tile_plans(n_qkv / 16, D, false, p.KS) : TilePlans{};
+}
+
 }  // namespace
 
 extern "C" size_t sf_qkv_workspace_bytes(int bucket, int D, int n_qkv) {
   if (bucket < 1 || D < kKC || D % kKC || n_qkv < 128 || n_qkv % 128) return 0;
-  return part_bytes(make_plan(n_qkv / 128, D / kKC), bucket, n_qkv);
+  const size_t a = part_bytes(qkv_plan(n_qkv, D), bucket, n_qkv);
+  // (never less than a stream-K split of the same shape takes)
+  const size_t b = part_bytes(make_plan(n_qkv / 128, D / kKC), bucket, n_qkv);
+  return a > b ? a : b;
 }
 
 extern "C" int sf_qkv_rope(const uint16_t* xn, const int32_t* rows, const int32_t* count,
@@ -103,9 +119,10 @@ extern "C" int sf_qkv_rope(const uint16_t* xn, const int32_t* rows, const int32_
   const int n_qkv = (H + 2 * Hkv) * hd;
   if (workspace_bytes < sf_qkv_workspace_bytes(bucket, D, n_qkv)) return SF_ERR_WORKSPACE;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const Plan p = make_plan(n_qkv / 128, D / kKC);
+  const Plan p = qkv_plan(n_qkv, D);
+  const TilePlans tp = qkv_tiles(p, n_qkv, D);
   float* part = reinterpret_cast<float*>(workspace);
-  launch_sk<1, kPart>(p, xn, rows, D, count, 0, bucket, w_qkv, nullptr, D, n_qkv, part, Epi{}, st);
+  launch_sk<1, kPart>(p, tp, xn, rows, D, count, 0, bucket, w_qkv, nullptr, D, n_qkv, part, Epi{}, st);
   dim3 g2(min(bucket, 128), (H + 2 * Hkv + 3) / 4);
   hipLaunchKernelGGL(sf_qkv_epilogue_kernel<false>, g2, dim3(256), 0, st, part, p, bucket, n_qkv, rows,
                      count, b_qkv, cos_tab, sin_tab, pos0, table_rows, q_scale, N, H, Hkv, q_buf,
@@ -137,9 +154,10 @@ extern "C" int sf_qkv_rope_branches(const uint16_t* xn, const int32_t* rows,
   const int n_qkv = (H + 2 * Hkv) * hd;
   if (workspace_bytes < sf_qkv_workspace_bytes(bucket, D, n_qkv)) return SF_ERR_WORKSPACE;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const Plan p = make_plan(n_qkv / 128, D / kKC);
+  const Plan p = qkv_plan(n_qkv, D);
+  const TilePlans tp = qkv_tiles(p, n_qkv, D);
   float* part = reinterpret_cast<float*>(workspace);
-  launch_sk<1, kPart>(p, xn, rows, D, count, 0, bucket, w_qkv, nullptr, D, n_qkv, part, Epi{}, st);
+  launch_sk<1, kPart>(p, tp, xn, rows, D, count, 0, bucket, w_qkv, nullptr, D, n_qkv, part, Epi{}, st);
   dim3 g2(min(bucket, 128), (H + 2 * Hkv + 3) / 4);
   hipLaunchKernelGGL(sf_qkv_epilogue_kernel<true>, g2, dim3(256), 0, st, part, p, bucket, n_qkv,
                      rows, count, b_qkv, cos_tab, sin_tab, pos0_branch, table_rows, q_scale_rows,
@@ -175,10 +193,11 @@ extern "C" int sf_qkv_rope_gated(const uint16_t* xn, const int8_t* rec, const in
   const int n_qkv = (H + 2 * Hkv) * hd;
   if (workspace_bytes < sf_qkv_workspace_bytes(bucket, D, n_qkv)) return SF_ERR_WORKSPACE;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const Plan p = make_plan(n_qkv / 128, D / kKC);
+  const Plan p = qkv_plan(n_qkv, D);
+  const TilePlans tp = qkv_tiles(p, n_qkv, D);
   float* part = reinterpret_cast<float*>(workspace);
   const GateIn gate{rec, par, B1, N, GateOut{f, src, rows, count, seg, segcnt, slot}};
-  launch_sk<1, kPart, true>(p, xn, nullptr, D, nullptr, 0, bucket, w_qkv, nullptr, D, n_qkv, part,
+  launch_sk<1, kPart, true>(p, tp, xn, nullptr, D, nullptr, 0, bucket, w_qkv, nullptr, D, n_qkv, part,
                             Epi{}, st, gate);
   dim3 g2(min(bucket, 128), (H + 2 * Hkv + 3) / 4);
   if (pos0_per_branch)
