@@ -28,7 +28,7 @@ constexpr int kThreads = 512; // 8 waves
 // kKC (K per stage), kLdsBudget and SFG_RING_MAX: sf_index.h
 
 // One ring stage of a workgroup of up to MB rows and WN weight tiles per wave:
-// the two 32-K chunks of the MB/16 A m tiles (1 KB per (chunk, m tile)), then
+// the MB/16 A m tiles (2 KB each: 16 rows of 64 K), then
 // every wave's WN weight fragments of its chunk (1 KB each, in lane order: the
 // packed layout).  Sizes in 16-byte words.  The ring holds as many stages as fit
 // kLdsBudget, at most SFG_RING_MAX.
@@ -54,10 +54,9 @@ struct Stage {
 
 // The fragments are read from the ring by sf_lds_read16, which the compiler does
 // not track, so it adds no wait for the copies in flight (the waits are
-// sf_wait_vm_barrier's and sf_lds_reads_done's).  A rows are 64 bytes per
-// tile row, whose four 16-byte units are XOR-swizzled — unit u of tile row r
-// sits at position u ^ a_swz(r), so the 16 lanes of a fragment read that share
-// a unit hit distinct banks.
+// sf_wait_vm_barrier's and sf_lds_reads_done's).  A tile rows are 128 bytes (the
+// stage's 64 K), their eight 16-byte units XOR-swizzled (a2_copy_unit): a copy of 8
+// rows takes whole cache lines, and the lanes of a fragment read hit distinct banks.
 template <int MB, int WN>
 struct Ring {
   sf_u32x4* slot[8];
@@ -66,13 +65,13 @@ struct Ring {
 // Rows handled by one workgroup of a launch whose row count is at most mcap.
 inline int row_block(int mcap) { return mcap <= 64 ? 64 : 128; }
 
-// The A fragments (NMT m tiles, 1 KB apart) and weight fragments (WN tiles, CPS KB
+// The A fragments (NMT m tiles, 2 KB apart) and weight fragments (WN tiles, CPS KB
 // apart: a tile's CPS chunk blocks follow each other) of K chunk C of a stage, read
 // from LDS without waiting (sf_lds_read16 with compile-time offsets).
 template <int NMT, int WN, int CPS = 2, int I = 0>
 SF_DEV void lds_fragments(sf_u32x4 (&f)[NMT + WN], sf_lds_off a_addr, sf_lds_off w_addr) {
   if constexpr (I < NMT) {
-    f[I] = sf_lds_read16<I * 1024>(a_addr);
+    f[I] = sf_lds_read16<I * 2048>(a_addr);
     lds_fragments<NMT, WN, CPS, I + 1>(f, a_addr, w_addr);
   } else if constexpr (I < NMT + WN) {
     f[I] = sf_lds_read16<(I - NMT) * CPS * 1024>(w_addr);
@@ -86,7 +85,7 @@ SF_DEV void lds_fragments(sf_u32x4 (&f)[NMT + WN], sf_lds_off a_addr, sf_lds_off
 // row table in LDS.
 //
 // Every operand goes to LDS by direct copies (global_load_lds, 16 bytes per lane,
-// 1 KB per instruction): per stage the 2*NMT A tile copies (chunk, m tile) dealt
+// 1 KB per instruction): per stage the 2*NMT A copies of 8 rows dealt
 // out over the 8 waves (copy q to wave q % 8; a wave with fewer real copies
 // repeats the last one — the same bytes to the same place — so every wave issues
 // DPW per stage), and each wave's own 2*WN weight fragments (two chunks per
@@ -109,24 +108,22 @@ SF_DEV void mainloop(const uint16_t* __restrict__ A, int lda, int mrows, const i
   using St = Stage<MB, WN>;
   constexpr int R = St::kRing;
   static_assert(R >= 3, "the ring needs three stages");
-  constexpr int kMT = MB / 16;
   constexpr int DPW = (2 * NMT + 7) / 8;
   constexpr bool kWR = St::kWReg;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wv = tid >> 6;
   const int slast = s1 - 1;
-  // this lane's part of each A tile copy: tile row lane/4, stored unit lane%4
-  // holding A unit a_copy_unit(lane) of the copy's 32-K chunk
+  // this lane's part of each A copy q (8 rows of the stage's 64 K): row 8q + lane/8,
+  // stored unit lane%8 holding A unit a2_copy_unit(lane)
   const uint16_t* asrc[DPW];
   int adst[DPW];   // first word of the copy in a slot
 #pragma unroll
   for (int j = 0; j < DPW; ++j) {
     const int q = a_copy(wv, j, NMT);
-    const int ch = q / NMT, mt = q - ch * NMT;
-    const int r = sf_imin(mt * 16 + (lane >> 2), mrows - 1);
-    asrc[j] = A + (size_t)rows[r] * lda + ch * 32 + a_copy_unit(lane) * 8;
-    adst[j] = (ch * kMT + mt) * 64;
+    const int r = sf_imin(q * 8 + (lane >> 3), mrows - 1);
+    asrc[j] = A + (size_t)rows[r] * lda + a2_copy_unit(lane) * 8;
+    adst[j] = q * 64;
   }
   const int wdst = St::kA + wv * WN * 128;   // this wave's weights: [tile][chunk][1 KB]
   // kWR: this lane's weight fragments of the stages in flight, [ring slot][tile][chunk]
@@ -151,9 +148,10 @@ SF_DEV void mainloop(const uint16_t* __restrict__ A, int lda, int mrows, const i
 #pragma unroll
   for (int j = 0; j < R - 1; ++j) issue(s0 + j, j);
 
-  // this lane's A fragment in chunk c of a stage: word a_read_word(lane) of tile
-  // (c, mt); its weight fragment: word `lane` of block (tile t, chunk c)
-  const sf_lds_off a_byte = (sf_lds_off)a_read_word(lane) * 16;
+  // this lane's A fragment in chunk c of a stage: word a2_read_word(lane, c) of tile
+  // mt; its weight fragment: word `lane` of block (tile t, chunk c)
+  const sf_lds_off a_byte[2] = {(sf_lds_off)a2_read_word(lane, 0) * 16,
+                                (sf_lds_off)a2_read_word(lane, 1) * 16};
   const sf_lds_off w_byte = (sf_lds_off)(wdst + lane) * 16;
   // the fragment reads and MFMAs of the stage in ring slot j
   auto compute = [&](int j) {
@@ -163,7 +161,7 @@ SF_DEV void mainloop(const uint16_t* __restrict__ A, int lda, int mrows, const i
     for (int c = 0; c < 2; ++c) {
       constexpr int kLW = kWR ? 0 : WN;   // weight fragments read from LDS
       sf_u32x4 f[NMT + kLW];
-      lds_fragments<NMT, kLW>(f, base + a_byte + c * kMT * 1024, base + w_byte + c * 1024);
+      lds_fragments<NMT, kLW>(f, base + a_byte[c], base + w_byte + c * 1024);
       sf_lds_reads_done(f);
 #pragma unroll
       for (int mt = 0; mt < NMT; ++mt)

@@ -39,7 +39,6 @@ void gemm_rows_kernel(const uint16_t* __restrict__ A, int M, const uint16_t* __r
   using St = RowsStage<RG, WN>;
   constexpr int R = St::kRing;
   static_assert(R >= 3, "the ring needs three stages");
-  constexpr int kMT = St::kMT;
   __shared__ sf_u32x4 ring[R * St::kWords];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -53,19 +52,19 @@ void gemm_rows_kernel(const uint16_t* __restrict__ A, int M, const uint16_t* __r
   const int rgrp = wv / St::kCG;
   const int cgrp = wv - rgrp * St::kCG;
 
-  // this wave's copies: lane L of an A copy brings row L/4 of its m tile (rows
-  // past M re-read row M - 1), A unit a_copy_unit(L) of the chunk; lane L of a
-  // weight copy brings lane L's fragment of its (tile, chunk) block
+  // this wave's copies: lane L of A copy q brings row 8q + L/8 (rows past M re-read
+  // row M - 1), A unit a2_copy_unit(L) of the stage's 64 K; lane L of a weight copy
+  // brings lane L's fragment of its (tile, chunk) block
   constexpr int CPS = St::kCPS;
+  static_assert(CPS == 2, "A copies take 64 K of a row");
   const uint16_t* asrc[St::kDA];
   int adst[St::kDA];
 #pragma unroll
   for (int j = 0; j < St::kDA; ++j) {
     const int cq = rows_a_copy(wv + 8 * j, St::kNA);
-    const int ch = rows_a_chunk(cq, kMT), mt = rows_a_mtile(cq, kMT);
-    const int r = sf_imin(mt * 16 + (lane >> 2), M - 1);
-    asrc[j] = A + (size_t)r * K + ch * 32 + a_copy_unit(lane) * 8;
-    adst[j] = (ch * kMT + mt) * 64;
+    const int r = sf_imin(cq * 8 + (lane >> 3), M - 1);
+    asrc[j] = A + (size_t)r * K + a2_copy_unit(lane) * 8;
+    adst[j] = cq * 64;
   }
   const uint16_t* wsrc[St::kDW];
   int wdst[St::kDW];
@@ -94,10 +93,11 @@ void gemm_rows_kernel(const uint16_t* __restrict__ A, int M, const uint16_t* __r
 #pragma unroll
     for (int tt = 0; tt < WN; ++tt) acc[i][tt] = sf_f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // this lane's A fragment of m tile rgrp*8 + i in chunk c: word a_read_word(lane)
-  // of A tile (c, mt); its weight fragment of tile cgrp*WN + tt: word `lane` of
+  // this lane's A fragment of m tile rgrp*8 + i in chunk c: word a2_read_word(lane, c)
+  // of the tile; its weight fragment of tile cgrp*WN + tt: word `lane` of
   // block (tile, c)
-  const sf_lds_off a_byte = (sf_lds_off)(rgrp * 8 * 64 + a_read_word(lane)) * 16;
+  const sf_lds_off a_byte[2] = {(sf_lds_off)(rgrp * 8 * 128 + a2_read_word(lane, 0)) * 16,
+                                (sf_lds_off)(rgrp * 8 * 128 + a2_read_word(lane, 1)) * 16};
   const sf_lds_off w_byte = (sf_lds_off)(St::kA + cgrp * WN * CPS * 64 + lane) * 16;
 #pragma unroll 1
   for (int sb = s0; sb < s1; sb += R) {
@@ -110,7 +110,7 @@ void gemm_rows_kernel(const uint16_t* __restrict__ A, int M, const uint16_t* __r
 #pragma unroll
         for (int c = 0; c < CPS; ++c) {
           sf_u32x4 f[8 + WN];
-          lds_fragments<8, WN, CPS>(f, base + a_byte + c * kMT * 1024, base + w_byte + c * 1024);
+          lds_fragments<8, WN, CPS>(f, base + a_byte[c], base + w_byte + c * 1024);
           sf_lds_reads_done(f);
 #pragma unroll
           for (int i = 0; i < 8; ++i)

@@ -93,12 +93,12 @@ using HeadTail = HeadShape<8, 2, 2, 4, 256>;
 using HeadMain128 = HeadShape<8, 1, 2, 4, 128>;
 using HeadTail128 = HeadShape<8, 2, 2, 4, 128>;
 
-// The X fragments of FG consecutive m tiles (1 KB apart) from LDS byte address a,
+// The X fragments of FG consecutive m tiles (2 KB apart) from LDS byte address a,
 // without waiting (sf_lds_read16 with compile-time offsets).
 template <int FG, int I = 0>
 SF_DEV void head_fragments(sf_u32x4 (&f)[FG], sf_lds_off a) {
   if constexpr (I < FG) {
-    f[I] = sf_lds_read16<I * 1024>(a);
+    f[I] = sf_lds_read16<I * 2048>(a);
     head_fragments<FG, I + 1>(f, a);
   }
 }
@@ -122,7 +122,6 @@ void head_kernel(const uint16_t* __restrict__ X, int Mo, int m0, HeadRows hr,
                  const uint16_t* __restrict__ W, int K, int t0, uint16_t* __restrict__ out,
                  long long ldo) {
   using Sh = HeadShape<NW, RG, WN, R, HR>;
-  constexpr int kHMT = Sh::kMT;
   constexpr int kHStageWords = Sh::kStageWords;
   constexpr int kHDA = Sh::kDA;
   constexpr int kHDB = Sh::kDB;
@@ -143,18 +142,16 @@ void head_kernel(const uint16_t* __restrict__ X, int Mo, int m0, HeadRows hr,
   const int S = K / kKC;
   const int slast = S - 1;
 
-  // X copies: copy q = wv + NW*j is (chunk q / kHMT, m tile q % kHMT); lane L
-  // brings pass row L/4 of the tile (rows past Mo re-read the last one), unit
-  // a_copy_unit(L), from its input row
+  // X copies: lane L of copy q = wv + NW*j brings pass row 8q + L/8 (rows past Mo
+  // re-read the last one), unit a2_copy_unit(L) of the stage's 64 K, from its input row
   const uint16_t* asrc[kHDA];
   int adst[kHDA];
 #pragma unroll
   for (int j = 0; j < kHDA; ++j) {
     const int q = wv + NW * j;
-    const int ch = q / kHMT, mt = q - ch * kHMT;
-    const int r = sf_imin(m0 + mt * 16 + (lane >> 2), Mo - 1);
-    asrc[j] = X + (size_t)head_in_row(r, hr) * K + ch * 32 + a_copy_unit(lane) * 8;
-    adst[j] = (ch * kHMT + mt) * 64;
+    const int r = sf_imin(m0 + q * 8 + (lane >> 3), Mo - 1);
+    asrc[j] = X + (size_t)head_in_row(r, hr) * K + a2_copy_unit(lane) * 8;
+    adst[j] = q * 64;
   }
   // this lane's weight streams: 16-column tiles t*TN/16 + cg*WN + tt
   const uint16_t* wsrc[kHWN];
@@ -192,9 +189,10 @@ void head_kernel(const uint16_t* __restrict__ X, int Mo, int m0, HeadRows hr,
 #pragma unroll
     for (int tt = 0; tt < kHWN; ++tt) acc[i][tt] = sf_f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // this lane's X fragment of m tile rg*NMT + i in chunk c: word a_read_word(lane)
-  // of tile (c, rg*NMT + i)
-  const sf_lds_off a_byte = (sf_lds_off)((rg * NMT) * 64 + a_read_word(lane)) * 16;
+  // this lane's X fragment of m tile rg*NMT + i in chunk c: word a2_read_word(lane, c)
+  // of the tile
+  const sf_lds_off a_byte[2] = {(sf_lds_off)(rg * NMT * 128 + a2_read_word(lane, 0)) * 16,
+                                (sf_lds_off)(rg * NMT * 128 + a2_read_word(lane, 1)) * 16};
   // stage s in ring slot j: wait for it (issued R - 1 stages ago: its X copies of
   // every wave -- the barrier -- and this wave's weights; no wave still reads slot
   // j - 1), issue stage s + R - 1 into slot j - 1, then its MFMAs, FG m tiles at
@@ -212,7 +210,7 @@ void head_kernel(const uint16_t* __restrict__ X, int Mo, int m0, HeadRows hr,
     constexpr int NG = 2 * NH;
     sf_u32x4 fb[2][FG];
     auto group_addr = [&](int gi) {
-      return base + a_byte + ((gi / NH) * kHMT + (gi % NH) * FG) * 1024;
+      return base + a_byte[gi / NH] + (gi % NH) * FG * 2048;
     };
     head_fragments<FG>(fb[0], group_addr(0));
 #pragma unroll
