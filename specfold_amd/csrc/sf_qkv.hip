@@ -83,11 +83,11 @@ __global__ __launch_bounds__(256) void sf_qkv_epilogue_kernel(
 // Each head's tile cut into whole K ranges (split plan, as FFN down) while the heads
 // are fewer than the grid: the same ranges for every head, so that the tile GEMM (more
 // than 128 rows) gives every row the streaming core's sums.  A range holds at least
-// three 64-K stages: shorter ones are all ring fill, and their partial slots cost the
+// two 64-K stages: shorter ones are all ring fill, and their partial slots cost the
 // epilogue more than the idle CUs do the GEMM.
 Plan qkv_plan(int n_qkv, int D) {
   const int T = n_qkv / 128, S = D / kKC;
-  return T < SFG_GRID ? make_plan_split(T, S, 3) : make_plan(T, S);
+  return T < SFG_GRID ? make_plan_split(T, S, 2) : make_plan(T, S);
 }
 TilePlans qkv_tiles(const Plan& p, int n_qkv, int D) {
   return p.KS ? make_tile_plans(n_qkv / 16, D, false, p.KS) : TilePlans{};
