@@ -77,7 +77,8 @@ const char* sf_status_string(int status);
  *     attends its rows: the workspace holds the range partials only; B1 <= 64.
  * 12: SF_GATE_DEFER_COMPACT and sf_qkv_rope_gated (the compaction in the QKV GEMM).
  * 13: sf_head_logits_rows (the head for the rows a decode step reads).
- * 14: sf_decode_facts; sf_attn_rows / sf_attn_prefix_block take NULL o32, m_tab, z_tab. */
+ * 14: sf_decode_facts; sf_attn_rows / sf_attn_prefix_block take NULL o32, m_tab, z_tab
+ *     (sf_attn_chunk joined it: an addition, nothing that was there changed). */
 int sf_abi_version(void);
 
 /*
@@ -245,6 +246,25 @@ int sf_attn_rows(const uint16_t* q_buf, const uint16_t* kv_buf, const uint16_t* 
                  int b_first, int b_count, int H, int Hkv, int hd, float scaling,
                  const int32_t* prefix_len, float* o32, uint16_t* o_bf, float* m_tab,
                  float* z_tab, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * (3) for a prompt's consecutive blocks at once: n rows whose K and V are in the cache
+ * already (sf_kv_append), row m at position P - n + m of the P cached tokens.  Row m
+ * attends to every key below the end of its own block of `block` rows (blocks counted
+ * from row 0, the last one may be short): the block-diffusion prefill of
+ * specfold/generate/fastdllm_v2_generation.py:510-524 (bidirectional in a block, causal
+ * across blocks); block = 1: causal (specfold/generate/nld_generation.py:186-194).
+ * Writes o_bf for rows 0 .. n - 1 (row stride H*hd).  Same softmax arithmetic as
+ * sf_attn_prefix_block.  workspace: sf_attn_chunk_workspace_bytes(n, H), 16-byte aligned.
+ * Limits: hd == 128, H % Hkv == 0, H/Hkv <= 8, 1 <= n <= 1024, n <= P <= 32768, the page
+ * sizes of sf_attn_prefix_block.  No counterpart in the reference, whose prefill is
+ * inside the checkpoint's remote code.
+ */
+size_t sf_attn_chunk_workspace_bytes(int n, int H);
+int sf_attn_chunk(const uint16_t* q_buf, const uint16_t* cache_k, const uint16_t* cache_v,
+                  const int32_t* page_table, int P, int page_size, long long page_stride,
+                  long long head_stride, int n, int block, int H, int Hkv, int hd, float scaling,
+                  uint16_t* o_bf, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * (4) Chain correction of folded rows: start from the state of the nearest

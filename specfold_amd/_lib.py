@@ -54,6 +54,9 @@ SIGNATURES = {
     "sf_attn_rows": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _ll, _ll, _vp, _vp, _vp,
                           _i, _i, _i, _i, _i, _i, _i, _i, _f, _vp, _vp, _vp, _vp, _vp, _vp,
                           _sz, _vp]),
+    "sf_attn_chunk_workspace_bytes": (_sz, [_i, _i]),
+    "sf_attn_chunk": (_i, [_vp, _vp, _vp, _vp, _i, _i, _ll, _ll, _i, _i, _i, _i, _i, _f, _vp, _vp,
+                           _sz, _vp]),
     "sf_chain_correct": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _f,
                               _vp, _vp, _vp, _vp, _vp]),
     "sf_kv_append": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _i, _ll, _ll, _i, _vp]),
@@ -405,6 +408,31 @@ def attn_rows(q_buf, kv_buf, prefix_k, prefix_v, page_table, P, page_size, page_
         _ptr(o32), _ptr(o_bf), _ptr(m_tab), _ptr(z_tab), _ptr(workspace), workspace.numel(),
         _stream(stream))
     _check(st, "sf_attn_rows")
+
+
+def attn_chunk_workspace_bytes(n: int, H: int) -> int:
+    return int(load().sf_attn_chunk_workspace_bytes(n, H))
+
+
+def attn_chunk(q_buf, cache_k, cache_v, page_table, P, page_size, page_stride, head_stride, n,
+               block, H, Hkv, hd, scaling, o_bf, workspace, stream=None) -> None:
+    """Attention of the n rows of consecutive blocks whose K/V are the last n of the P
+    cached tokens: every row sees the keys below its own block's end (block = 1:
+    causal)."""
+    _need(q_buf, "q_buf", torch.bfloat16, min_numel=n * H * hd)
+    _need(cache_k, "cache_k", torch.bfloat16)
+    _need(cache_v, "cache_v", torch.bfloat16)
+    if page_table is not None:
+        _need(page_table, "page_table", torch.int32, min_numel=(P + page_size - 1) // page_size,
+              align=4)
+    _need(o_bf, "o_bf", torch.bfloat16, min_numel=n * H * hd)
+    _need(workspace, "workspace", torch.uint8, min_numel=attn_chunk_workspace_bytes(n, H),
+          align=256)
+    st = load().sf_attn_chunk(_ptr(q_buf), _ptr(cache_k), _ptr(cache_v), _ptr(page_table), P,
+                              page_size, page_stride, head_stride, n, block, H, Hkv, hd,
+                              float(scaling), _ptr(o_bf), _ptr(workspace), workspace.numel(),
+                              _stream(stream))
+    _check(st, "sf_attn_chunk")
 
 
 def chain_correct(q_buf, kv_buf, src, par, rec, seg, segcnt, B1, N, H, Hkv, hd, scaling,

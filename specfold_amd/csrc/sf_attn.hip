@@ -93,13 +93,26 @@ SF_DEV void pv_parts(const float (&p)[2][4], sf_bf16x8 (&b)[NP]) {
   for (int i = 0; i < NP; ++i) b[i] = sf_as_bf16x8(w[i]);
 }
 
+// The rows of several consecutive blocks whose keys are in the cache too
+// (sf_attn_chunk): n rows, row m at position P - n + m of the P cached keys; it sees
+// the keys below own_limit (its own block's end; blk = 1: causal).  direct: one range
+// per query, the output is written from here (o_bf).
+struct OwnRows {
+  int n, blk, direct;
+  uint16_t* o_bf;
+};
+SF_DEV int own_limit(int m, int P, const OwnRows& own) {
+  return P - own.n + min(own.n, (m / own.blk + 1) * own.blk);
+}
+
+template <bool OWN>
 SF_DEV void prefix_item(const uint16_t* __restrict__ q_buf, const uint16_t* __restrict__ pk,
                         const uint16_t* __restrict__ pv, const int32_t* __restrict__ page_table,
                         int page_size, long long page_stride, long long head_stride, int P,
                         const int32_t* __restrict__ rows, int nq, int G, int H, float scale_log2,
                         int qmax, int nr_cap, int qt, int r, int c0, int c1, int h,
                         uint8_t* ring, int* s_pg, float* __restrict__ ws_o,
-                        float* __restrict__ ws_ml) {
+                        float* __restrict__ ws_ml, const OwnRows& own) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wv = tid >> 6;
@@ -120,12 +133,14 @@ SF_DEV void prefix_item(const uint16_t* __restrict__ q_buf, const uint16_t* __re
       s_pg[i] = page_table[chunk_group_g0(c0 + (i >> 2), i & 3, last_g0) / page_size];
   }
   int qrow[2], qhead[2];
+  int lim[2];   // OWN: the keys each query sees
 #pragma unroll
   for (int qs = 0; qs < 2; ++qs) {
     // a padding query (qi >= nq) repeats the last real one; its partial is not written
     const int qc = min(qt * kQT + qg * 32 + qs * 16 + ql, nq - 1);
     const int m = qc / G;
-    qrow[qs] = rows[m];
+    qrow[qs] = OWN ? m : rows[m];
+    lim[qs] = OWN ? own_limit(m, P, own) : P;
     qhead[qs] = h * G + (qc - m * G);
   }
   sf_wait_vm_loads();
@@ -306,14 +321,15 @@ SF_DEV void prefix_item(const uint16_t* __restrict__ q_buf, const uint16_t* __re
     sf_u32x2 vf[16];
     read_vt(vbase, vf);
     const int kbase = c * kChunk + kh * 32 + grp * 4;  // key of s[0][.][0] of this lane
-    if (kbase + 16 + 3 >= P) {  // a partial last chunk: keys past the prefix
+    // a partial last chunk: keys past the prefix (OWN: past the query's limit)
+    if (kbase + 16 + 3 >= (OWN ? min(lim[0], lim[1]) : P)) {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int qs = 0; qs < 2; ++qs)
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            if (kbase + 16 * t + i >= P) s[t][qs][i] = -INFINITY;
+            if (kbase + 16 * t + i >= (OWN ? lim[qs] : P)) s[t][qs][i] = -INFINITY;
     }
 
     // online softmax per query (base 2, scores pre-scaled by log2(e) * scaling).
@@ -446,10 +462,29 @@ SF_DEV void prefix_item(const uint16_t* __restrict__ q_buf, const uint16_t* __re
       const float m1 = xml[((qg * 2 + qs) * 16 + ql) * 4];
       const float l1 = xml[((qg * 2 + qs) * 16 + ql) * 4 + 1];
       const float h1 = xml[((qg * 2 + qs) * 16 + ql) * 4 + 2];
-      const float mm = fmaxf(m_hi[qs], h1);  // finite: half 0 holds the range's first key
+      // finite: half 0 holds the range's first key (OWN: a query may see no key of the
+      // range; its weights are then 0)
+      float mm = fmaxf(m_hi[qs], h1);
+      if (OWN && mm == -INFINITY) mm = 0.f;
       const float w0 = __builtin_amdgcn_exp2f(m_ref[qs] - mm);
       const float w1 = __builtin_amdgcn_exp2f(m1 - mm);
-      if (qi < nq) {
+      if (OWN && own.direct) {   // (an argument: workgroup-uniform)
+        if (qi < nq) {
+          const float inv = 1.0f / (l_run[qs] * w0 + l1 * w1);
+          const int m = qi / G;
+          uint16_t* op = own.o_bf + (size_t)m * H * kHD + (h * G + (qi - m * G)) * kHD + grp * 4;
+#pragma unroll
+          for (int dt = 0; dt < 8; ++dt) {
+            const sf_f32x4 a1 =
+                *reinterpret_cast<const sf_f32x4*>(xo + (((qg * 2 + qs) * 8 + dt) * 64 + lane) * 4);
+            const sf_f32x4 o = (acc[qs][dt] * w0 + a1 * w1) * inv;
+            sf_u32x2 w;
+            w[0] = sf_pack2(o[0], o[1]);
+            w[1] = sf_pack2(o[2], o[3]);
+            sf_handoff_store(reinterpret_cast<sf_u32x2*>(op + dt * 16), w);
+          }
+        }
+      } else if (qi < nq) {
         const size_t slot = attn_slot(h, r, qi, nr_cap, qmax);
         if (grp == 0) {
           sf_handoff_store(reinterpret_cast<sf_f32x2*>(ws_ml + slot * 2),
@@ -492,11 +527,85 @@ sf_attn_prefix_kernel(
   for (int it = xcd_begin(items, xcd) + (int)(blockIdx.x >> 3); it < end; it += per) {
     const AttnItem item = attn_item(it, pg.n_qt, pg.nr);
     const int c0 = item.r * pg.cpi;
-    prefix_item(q_buf, pk, pv, page_table, page_size, page_stride, head_stride, P, rows, nq, G, H,
-                scale_log2, qmax, nr_cap, item.qt, item.r, c0, min(pg.nch, c0 + pg.cpi), item.h,
-                ring, s_pg, ws_o, ws_ml);
+    prefix_item<false>(q_buf, pk, pv, page_table, page_size, page_stride, head_stride, P, rows, nq,
+                       G, H, scale_log2, qmax, nr_cap, item.qt, item.r, c0,
+                       min(pg.nch, c0 + pg.cpi), item.h, ring, s_pg, ws_o, ws_ml, OwnRows{});
     __syncthreads();  // LDS is reused by the next item
   }
+}
+
+// ---- rows of several blocks at once, their own keys in the cache (sf_attn_chunk) ---------
+// A prompt's blocks used to go through the model one at a time, 32 rows a forward; all
+// of them (up to 1024 rows) share a forward when each row is held to its own block's end
+// here.  The same items as the prefix pass -- (query tile of 128, range of cpi chunks, kv
+// head) -- over the P cached keys, the block's own among them; an item stops at the
+// last key its tile sees, and a range past it is no item.  Items are dealt out round
+// robin, the tiles with the most keys first, so that the triangle over the own keys
+// evens out.  Bound by the chunk step's MFMA + softmax + LDS reads, as the prefix pass.
+__global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+sf_attn_chunk_kernel(const uint16_t* __restrict__ q_buf, const uint16_t* __restrict__ pk,
+                     const uint16_t* __restrict__ pv, const int32_t* __restrict__ page_table,
+                     int page_size, long long page_stride, long long head_stride, int P, int H,
+                     int Hkv, float scale_log2, int nr, int cpi, OwnRows own,
+                     float* __restrict__ ws_o, float* __restrict__ ws_ml) {
+  __shared__ __attribute__((aligned(16))) uint8_t ring[kRing * kSlotBytes];
+  __shared__ int s_pg[4 * kMaxChunks];
+  const int G = H / Hkv;
+  const int nq = own.n * G;
+  const int n_qt = (nq + kQT - 1) / kQT;
+  const int items = n_qt * nr * Hkv;
+  for (int it = blockIdx.x; it < items; it += gridDim.x) {
+    const int qt = n_qt - 1 - it % n_qt;
+    const int rest = it / n_qt;
+    const int r = rest % nr, h = rest / nr;
+    const int nch = (own_limit((min(nq, (qt + 1) * kQT) - 1) / G, P, own) + kChunk - 1) / kChunk;
+    const int c0 = r * cpi;
+    if (c0 >= nch) continue;   // workgroup-uniform
+    prefix_item<true>(q_buf, pk, pv, page_table, page_size, page_stride, head_stride, P, nullptr,
+                      nq, G, H, scale_log2, nq, nr, qt, r, c0, min(nch, c0 + cpi), h, ring, s_pg,
+                      ws_o, ws_ml, own);
+    __syncthreads();  // LDS is reused by the next item
+  }
+}
+
+// o[m][hq] from the ranges that hold a key of row m: one wave per (row, q-head), two
+// dims per lane, the ranges' partials four at a time.
+__global__ __launch_bounds__(256) void sf_attn_chunk_merge_kernel(
+    int P, int H, int Hkv, int nr, int cpi, OwnRows own, const float* __restrict__ ws_o,
+    const float* __restrict__ ws_ml) {
+  const int lane = threadIdx.x & 63;
+  const int e = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (e >= own.n * H) return;
+  const int m = e / H, hq = e - m * H;
+  const int G = H / Hkv;
+  const int h = hq / G;
+  const int qmax = own.n * G;
+  const int qi = m * G + (hq - h * G);
+  const int nch = (own_limit(m, P, own) + kChunk - 1) / kChunk;
+  const int nm = (nch + cpi - 1) / cpi;   // <= nr: every one holds a key of the row
+  const size_t slot0 = attn_slot(h, 0, qi, nr, qmax);
+  const sf_f32x2 ml = sf_handoff_load(reinterpret_cast<const sf_f32x2*>(
+      ws_ml + (slot0 + (size_t)min(lane, nm - 1) * qmax) * 2));
+  const float mr = lane < nm ? ml.x : -INFINITY;
+  const float mm = sf_wave_max(mr);
+  const float w = lane < nm ? __builtin_amdgcn_exp2f(mr - mm) : 0.f;
+  const float inv = 1.0f / sf_wave_sum(ml.y * w);
+  float ax = 0.f, ay = 0.f;
+  for (int r0 = 0; r0 < nm; r0 += 4) {
+    sf_f32x2 a[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      a[u] = sf_handoff_load(reinterpret_cast<const sf_f32x2*>(
+          ws_o + (slot0 + (size_t)min(r0 + u, nm - 1) * qmax) * kHD + 2 * lane));
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float wr = __shfl(w, min(r0 + u, 63), 64);   // 0 past nm
+      ax = fmaf(wr, a[u].x, ax);
+      ay = fmaf(wr, a[u].y, ay);
+    }
+  }
+  *reinterpret_cast<uint32_t*>(own.o_bf + ((size_t)m * H + hq) * kHD + 2 * lane) =
+      sf_pack2(ax * inv, ay * inv);
 }
 
 // ---- rows: the prefix merge and the block attention, per source row ---------------------
@@ -907,4 +1016,64 @@ extern "C" int sf_attn_rows(const uint16_t* q_buf, const uint16_t* kv_buf,
                    head_stride, src, rows, count, bucket, B1, N, b_first, b_count, H, Hkv, hd,
                    scaling, prefix_len, 0, o32, o_bf, m_tab, z_tab, workspace, workspace_bytes,
                    reinterpret_cast<hipStream_t>(stream));
+}
+
+namespace {
+// Ranges a query's keys are cut into: as many as shorten the longest workgroup's share
+// (whole items of nch / nr chunks, about three chunks' time of set-up and partials
+// each), within the workspace of chunk_ranges_cap(n).
+int chunk_ranges_cap(int n) { return n >= 1024 ? 4 : (n <= 256 ? 16 : 4096 / n); }
+int chunk_ranges(int n, int P, int H, int Hkv) {
+  const int tiles = (n * (H / Hkv) + kQT - 1) / kQT * Hkv;
+  const int nch = nchunks_for(P);
+  int best = 1;
+  long long cost = -1;
+  for (int nr = 1; nr <= chunk_ranges_cap(n) && nr <= nch; ++nr) {
+    const long long c = (long long)((tiles * nr + kCUs - 1) / kCUs) * ((nch + nr - 1) / nr + 3);
+    if (cost < 0 || c < cost) {
+      cost = c;
+      best = nr;
+    }
+  }
+  return best;
+}
+}  // namespace
+
+extern "C" size_t sf_attn_chunk_workspace_bytes(int n, int H) {
+  if (n < 1 || n > kMaxBucket || H < 1) return 0;
+  return (size_t)chunk_ranges_cap(n) * n * H * (kHD + 2) * sizeof(float);
+}
+
+extern "C" int sf_attn_chunk(const uint16_t* q_buf, const uint16_t* cache_k,
+                             const uint16_t* cache_v, const int32_t* page_table, int P,
+                             int page_size, long long page_stride, long long head_stride, int n,
+                             int block, int H, int Hkv, int hd, float scaling, uint16_t* o_bf,
+                             void* workspace, size_t workspace_bytes, void* stream) {
+  if (!q_buf || !cache_k || !cache_v || !o_bf || !workspace) return SF_ERR_ARG;
+  if (hd != kHD || H < 1 || Hkv < 1 || H % Hkv != 0 || H / Hkv > kMaxG) return SF_ERR_SHAPE;
+  if (n < 1 || n > kMaxBucket || block < 1 || P < n || nchunks_for(P) > kMaxChunks)
+    return SF_ERR_SHAPE;
+  if (page_table && (page_size < 16 || page_size > 128 || (page_size & (page_size - 1))))
+    return SF_ERR_SHAPE;
+  if (!page_table && head_stride < (long long)P * kHD) return SF_ERR_SHAPE;
+  if (workspace_bytes < sf_attn_chunk_workspace_bytes(n, H)) return SF_ERR_WORKSPACE;
+  if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0) return SF_ERR_ARG;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const int nch = nchunks_for(P);
+  int nr = chunk_ranges(n, P, H, Hkv);
+  const int cpi = (nch + nr - 1) / nr;
+  nr = (nch + cpi - 1) / cpi;
+  const OwnRows own{n, block, nr == 1 ? 1 : 0, o_bf};
+  const int qmax = n * (H / Hkv);
+  float* ws_o = reinterpret_cast<float*>(workspace);
+  float* ws_ml = ws_o + (size_t)nr * qmax * Hkv * kHD;
+  const int items = (qmax + kQT - 1) / kQT * nr * Hkv;
+  hipLaunchKernelGGL(sf_attn_chunk_kernel, dim3(items < kCUs ? items : kCUs),
+                     dim3(kPrefixThreads), 0, st, q_buf, cache_k, cache_v, page_table, page_size,
+                     page_stride, head_stride, P, H, Hkv, scaling * 1.44269504088896340736f, nr,
+                     cpi, own, ws_o, ws_ml);
+  if (nr > 1)
+    hipLaunchKernelGGL(sf_attn_chunk_merge_kernel, dim3((n * H + 3) / 4), dim3(256), 0, st, P, H,
+                       Hkv, nr, cpi, own, ws_o, ws_ml);
+  return sf_launch_status();
 }

@@ -175,6 +175,39 @@ class _Buffers:
                                     dtype=torch.uint8, device=dev)
 
 
+class _ChunkBuffers:
+    """Device buffers of a cache-filling forward of up to ``cap`` consecutive rows
+    (FoldedVerifyEngine.append_blocks); reused across calls."""
+
+    def __init__(self, eng: "FoldedVerifyEngine", cap: int):
+        dev, bf = eng.device, torch.bfloat16
+        D, H, Hkv, hd = eng.D, eng.H, eng.Hkv, eng.hd
+        nq = (H + 2 * Hkv) * hd
+        i32 = dict(dtype=torch.int32, device=dev)
+        self.rec = torch.zeros(cap, dtype=torch.int8, device=dev)
+        self.f, self.src, self.rows, self.seg, self.slot = (torch.zeros(cap, **i32)
+                                                            for _ in range(5))
+        self.count, self.segcnt, self.par = (torch.zeros(1, **i32) for _ in range(3))
+        self.rstd = torch.empty(cap, dtype=torch.float32, device=dev)
+        self.hid = torch.empty(2, cap, D, dtype=bf, device=dev)
+        self.xn, self.zn, self.final = (torch.empty(cap, D, dtype=bf, device=dev)
+                                        for _ in range(3))
+        self.hp, self.ffn = (torch.empty(cap + 1, D, dtype=bf, device=dev) for _ in range(2))
+        self.q_buf = torch.empty(cap + 1, H * hd, dtype=bf, device=dev)
+        self.kv_buf = torch.empty(cap + 1, 2 * Hkv * hd, dtype=bf, device=dev)
+        self.o_bf = torch.empty(cap, H * hd, dtype=bf, device=dev)
+        self.act = torch.empty(cap, eng.I, dtype=bf, device=dev)
+        # the kernels of a layer run one after the other: one workspace for all
+        self.ws = torch.empty(max(_lib.gemm_workspace_bytes(cap, D, eng.I),
+                                  _lib.gate_up_workspace_bytes(cap, D, eng.I),
+                                  _lib.qkv_workspace_bytes(cap, D, nq),
+                                  *(_lib.o_proj_workspace_bytes(m, D, H * hd)
+                                    for m in (128, 256, cap)),
+                                  *(_lib.attn_chunk_workspace_bytes(m, H)
+                                    for m in (256, cap)), 256),
+                              dtype=torch.uint8, device=dev)
+
+
 class _Batch:
     """Several sequences' branch trees stacked into one verify step: sequence s
     owns branches offsets[s] .. offsets[s] + sizes[s] - 1 (its main branch first)
@@ -289,6 +322,7 @@ class FoldedVerifyEngine:
         del w
         self.head_kernel = "hip"
         self._bufs: Dict[Tuple[int, int, int], _Buffers] = {}
+        self._chunk_bufs: Dict[int, _ChunkBuffers] = {}   # by capacity: powers of two to 1024
         # HIP graphs of the layer loop, keyed by shape / prefix / delta / cache
         # (one per branch count the decode loop visits, B1 = 1..8, per sequence's
         # cache: several sequences decoded in turn each keep their own set)
@@ -439,6 +473,106 @@ class FoldedVerifyEngine:
             return None
         rows = None if head_rows is None else (N, int(head_rows[0]), int(head_rows[1]))
         return self.lm_head(buf.final, shift_n=N if shift else 0, rows=rows).view(B1, N, self.V)
+
+    # rows of one append_blocks forward (the kernels' row limit) and keys of a prefix
+    CHUNK_ROWS = 1024
+    MAX_KEYS = 32768
+
+    @torch.no_grad()
+    def append_blocks(self, tokens: torch.Tensor, cache: PagedKVCache, block: int,
+                      causal: bool = False, q_scale: Optional[torch.Tensor] = None,
+                      out: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """Cache-filling forward of consecutive blocks: tokens [1, n] (n <= CHUNK_ROWS) of
+        ``block`` tokens each (the last may be short) through every layer at once, every
+        row recomputed, their K/V appended to ``cache`` -> unshifted logits [n, V] (in
+        ``out``, [n, V_pad] bf16, if given).  The result of ``forward(..., append=True)``
+        block after block -- a row sees the cached keys and its own and earlier blocks'
+        (``causal``: itself and earlier rows) -- with the weights read once per
+        CHUNK_ROWS rows instead of once per block.  q_scale: fp32 [n]."""
+        n = tokens.shape[1]
+        if tokens.shape[0] != 1 or not 1 <= n <= self.CHUNK_ROWS or not 1 <= block <= 64:
+            raise ValueError("append_blocks takes [1, n] tokens, n <= "
+                             f"{self.CHUNK_ROWS}, in blocks of at most 64")
+        if not isinstance(cache, PagedKVCache):
+            raise TypeError("append_blocks needs a PagedKVCache")
+        P = cache.length
+        if P + n > min(cache.capacity, self.MAX_KEYS):
+            raise ValueError(f"KV cache full: {P}+{n} > capacity {cache.capacity}")
+        tokens = tokens.to(self.device).contiguous()
+        cap = max(64, 1 << (n - 1).bit_length())
+        buf = self._chunk_bufs.get(cap)
+        if buf is None:
+            buf = self._chunk_bufs[cap] = _ChunkBuffers(self, cap)
+        cos, sin = self.rope_tables(P + n)
+        if q_scale is not None:
+            q_scale = q_scale.reshape(-1).to(device=self.device, dtype=torch.float32).contiguous()
+        H, Hkv, hd, D = self.H, self.Hkv, self.hd, self.D
+        mode = _lib.SF_GATE_ALL | _lib.SF_GATE_DEFER_COMPACT
+        hidden = self.base.embed_tokens(tokens).reshape(n, D).contiguous()
+        for li, lyr in enumerate(self.layers):
+            ln_w = lyr.input_layernorm.weight
+            if li == 0:
+                _lib.fold_gate(hidden, buf.par, ln_w, 1, n, n, 0.0, self.eps, mode, buf.rec,
+                               buf.f, buf.src, buf.rows, buf.count, buf.seg, buf.segcnt, buf.rstd,
+                               buf.xn, slot=buf.slot)
+            else:
+                hidden = buf.hid[li % 2]
+                _lib.fold_gate_residual(buf.hp, buf.ffn, buf.src, buf.par, ln_w, 1, n, D, n, 0.0,
+                                        self.eps, mode, hidden, buf.rec, buf.f, buf.src, buf.rows,
+                                        buf.count, buf.seg, buf.segcnt, buf.slot, buf.rstd, buf.xn)
+            w_qkv, b_qkv = self._packed[li]
+            _lib.qkv_rope_gated(buf.xn, buf.rec, buf.par, 1, n, n, buf.f, buf.src, buf.rows,
+                                buf.count, buf.seg, buf.segcnt, buf.slot, w_qkv, b_qkv, cos, sin,
+                                q_scale, D, H, Hkv, hd, buf.q_buf, buf.kv_buf, buf.ws,
+                                pos0=cache.length_dev)
+            cache.append_rows(li, buf.kv_buf, 0, n)
+            v = cache.view(li)
+            _lib.attn_chunk(buf.q_buf, v.k, v.v, v.page_table, P + n, v.page_size, v.page_stride,
+                            v.head_stride, n, 1 if causal else block, H, Hkv, hd, self.scaling,
+                            buf.o_bf, buf.ws)
+            _lib.o_proj_post_norm(buf.o_bf, hidden, self._packed_o[li], n, H * hd, D, buf.slot,
+                                  lyr.post_attention_layernorm.weight, self.eps, buf.hp, buf.zn,
+                                  buf.ws)
+            wg, wu, wd = self._packed_mlp[li]
+            _lib.ffn_gate_up(buf.zn, buf.count, n, wg, wu, D, self.I, buf.act, buf.ws)
+            _lib.ffn_down_scatter(buf.act, buf.count, n, buf.rows, wd, self.I, D, buf.ffn, buf.ws)
+        last = buf.hid[self.L % 2]
+        _lib.residual_rmsnorm(buf.hp, buf.ffn, buf.src, self.base.norm.weight, 1, n, D, self.eps,
+                              last, buf.final)
+        cache.advance(n)
+        self.last_hidden = last[:n]
+        return self.lm_head(buf.final[:n], out=out)
+
+    @torch.no_grad()
+    def append_prompt(self, tokens: torch.Tensor, cache: PagedKVCache, block: int,
+                      causal: bool = False, q_scale=None) -> torch.Tensor:
+        """A prompt's blocks appended to ``cache`` -> unshifted logits [1, L, V], as
+        ``forward(..., append=True)`` block after block.  Runs of blocks go through
+        ``append_blocks``; a single block, and whatever that cannot take (a cache too
+        small for the run), one block at a time.  q_scale(P, n): the per-position q scale
+        of n positions from P (fp32 [n] or None), or None."""
+        L = tokens.shape[1]
+        per = self.CHUNK_ROWS // block * block if 1 <= block <= 64 else 0
+        fits = cache.length + L <= min(cache.capacity, self.MAX_KEYS)
+        if not per or L <= block or not fits:
+            prev_mode, self.gate_mode = self.gate_mode, _lib.SF_GATE_ALL
+            try:
+                parts = []
+                for s in range(0, L, block):
+                    blk = tokens[:, s:s + block]
+                    qs = None if q_scale is None else q_scale(cache.length, blk.shape[1])
+                    parts.append(self.forward(blk, cache, delta=0.0, append=True, q_scale=qs,
+                                              causal=causal))
+            finally:
+                self.gate_mode = prev_mode
+            return parts[0].contiguous() if len(parts) == 1 else torch.cat(parts, dim=1)
+        logits = torch.empty(L, self.V_pad, dtype=torch.bfloat16, device=self.device)
+        for s in range(0, L, per):
+            blk = tokens[:, s:s + per]
+            n = blk.shape[1]
+            qs = None if q_scale is None else q_scale(cache.length, n)
+            self.append_blocks(blk, cache, block, causal=causal, q_scale=qs, out=logits[s:s + n])
+        return logits[:, :self.V].contiguous().view(1, L, self.V)
 
     @torch.no_grad()
     def forward_batched(self, blocks: List[torch.Tensor], caches: list, delta: float = 0.1,

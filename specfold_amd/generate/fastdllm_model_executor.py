@@ -91,17 +91,8 @@ class FastDLLMModelExecutor:
             cache = past_key_values if past_key_values is not None else self.new_cache()
             if not isinstance(cache, PagedKVCache):
                 raise TypeError("update_past_key_values needs a PagedKVCache")
-            L = input_seq.shape[1]
-            bl = self.block_length
-            logits = []
-            for s in range(0, L, bl):
-                blk = input_seq[:, s:s + bl]
-                prev_mode, eng.gate_mode = eng.gate_mode, _lib.SF_GATE_ALL
-                try:
-                    logits.append(eng.forward(blk, cache, delta=0.0, append=True))
-                finally:
-                    eng.gate_mode = prev_mode
-            return SimpleNamespace(logits=torch.cat(logits, dim=1), past_key_values=cache)
+            logits = eng.append_prompt(input_seq, cache, self.block_length)
+            return SimpleNamespace(logits=logits, past_key_values=cache)
         prev_mode, eng.gate_mode = eng.gate_mode, _lib.SF_GATE_ALL
         try:
             logits = eng.forward(input_seq, past_key_values, delta=0.0)

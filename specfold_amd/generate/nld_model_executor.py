@@ -119,14 +119,9 @@ class NLDModelExecutor:
                 cache = past_key_values if past_key_values is not None else self.new_cache()
                 if not isinstance(cache, PagedKVCache):
                     raise TypeError("use_cache needs a PagedKVCache")
-                L = input_seq.shape[1]
-                logits = []
-                for s in range(0, L, self.block_length):
-                    blk = input_seq[:, s:s + self.block_length]
-                    qs = self.q_scale(cache.length, blk.shape[1])
-                    logits.append(eng.forward(blk, cache, delta=0.0, append=True, q_scale=qs,
-                                              causal=causal))
-                return SimpleNamespace(logits=torch.cat(logits, dim=1), past_key_values=cache)
+                logits = eng.append_prompt(input_seq, cache, self.block_length, causal=causal,
+                                           q_scale=self.q_scale)
+                return SimpleNamespace(logits=logits, past_key_values=cache)
             qs = self.q_scale(cache_length(past_key_values), input_seq.shape[1])
             logits = eng.forward(input_seq, past_key_values, delta=0.0, q_scale=qs, causal=causal)
             return SimpleNamespace(logits=logits, past_key_values=past_key_values)

@@ -9,7 +9,7 @@ import torch
 import torch.nn.functional as F
 
 from specfold_amd import _lib
-from test_gpu_gemm import acc_bound, close_bf16, mm64, packed, rnd, zeros_ws
+from tests.test_gpu_gemm import acc_bound, close_bf16, mm64, packed, rnd, zeros_ws
 
 pytestmark = pytest.mark.gpu
 

@@ -7,7 +7,7 @@ import subprocess
 
 import pytest
 
-from test_sim_gemm import _build
+from tests.test_sim_gemm import _build
 
 
 @pytest.fixture(scope="module")
