@@ -423,14 +423,32 @@ extern "C" size_t sf_o_proj_workspace_bytes(int M, int N, int K) {
 }
 
 namespace {
+// More than 256 rows: the tile GEMM over the all-rows GEMM's K ranges (the same sums, bit
+// for bit), one launch for every row instead of one per 256, each with its own ring
+// fill and drain.  o_proj + residual + norm, 320 / 640 / 1024 rows: 33.8 / 51.4 / 71.1 ->
+// 26.7 / 43.7 / 56.4 us at 3584, 54.2 / 81.2 / 111.8 -> 41.0 / 63.4 / 81.1 at 5120.  At 129 to 256 rows
+// (one launch either way) the all-rows GEMM's narrower tiles are 1-10 % faster.
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void o_proj_tile_kernel(const uint16_t* __restrict__ A, int M, const uint16_t* __restrict__ W,
+                        int K, int N, TilePlans tp, float* __restrict__ part) {
+  __shared__ sf_u32x4 ring[kLdsBudget / 16];
+  auto in_row = [](int r) { return r; };
+  tile_gemm<false>(TileGemm{A, K, W, nullptr, K, N / 16}, M, tp, ring, in_row,
+                   TilePartStore{part, M, N});
+}
+
 // o_proj over every row to the workspace's partial slots, then one wave per row
 // adds them to the residual (and normalises the recomputed rows when zn is given)
 int o_proj_launch(const uint16_t* o_bf, const uint16_t* x, const uint16_t* wo, int M, int K, int N,
                   const int32_t* slot, const uint16_t* ln_w, float eps, uint16_t* hp,
                   uint16_t* zn, void* workspace, hipStream_t st) {
   float* part = reinterpret_cast<float*>(workspace);
-  launch_rows<1, kRowsPart>(o_bf, M, wo, K, N, kOprojMaxSplits, part, nullptr, st);
   const int ks = rows_splits<1>(M, N, K, kOprojMaxSplits);
+  if (M > 256)
+    hipLaunchKernelGGL(o_proj_tile_kernel, dim3(SFG_GRID), dim3(kThreads), 0, st, o_bf, M, wo, K, N,
+                       make_tile_plans(N / 16, K, false, ks), part);
+  else
+    launch_rows<1, kRowsPart>(o_bf, M, wo, K, N, kOprojMaxSplits, part, nullptr, st);
   const size_t stride = (size_t)M * N;
   const int vpt = (N / 8 + kPrnThreads - 1) / kPrnThreads;
   const dim3 grid(M);
