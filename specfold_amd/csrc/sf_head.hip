@@ -34,6 +34,7 @@
 
 #include "sf_common.h"
 #include "sf_index.h"
+#include "sf_gemm_tile.h"
 
 namespace {
 
@@ -258,6 +259,57 @@ void head_kernel(const uint16_t* __restrict__ X, int Mo, int m0, HeadRows hr,
   }
 }
 
+// The head on the tile GEMM: 256-column tiles (the last partial round in 128-column
+// ones), the store's row map doing the window and the shift.  The sums are the kernel's
+// above bit for bit (K ascending in one accumulator).  Its cost follows the row blocks
+// (192 or 256 rows each, several in one launch), where the kernel above pays a whole
+// pass over the weights per 256 rows whatever they hold.
+//
+struct HeadTileStore {
+  HeadRows hr;
+  uint16_t* out;
+  long long ldo;
+  int units;
+  template <int NMT, int NT>
+  SF_DEV void operator()(int m0, int mrows, int, int u0, int rgrp, int cg,
+                         const sf_f32x4 (&acc)[NMT][NT]) const {
+    int lane = threadIdx.x & 63;
+    sf_pin(lane);   // nothing of the epilogue is hoisted over the item's main loop
+#pragma unroll
+    for (int i = 0; i < NMT; ++i) {
+      const int m = (rgrp * NMT + i) * 16 + (lane & 15);
+      if (m < mrows) {
+        uint16_t* p = out + (size_t)head_out_row(m0 + m, hr) * ldo + (lane >> 4) * 4;
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt) {
+          const int unit = u0 + cg * NT + tt;
+          if (unit < units) {
+            sf_u32x2 v;
+            v[0] = sf_pack2(acc[i][tt][0], acc[i][tt][1]);
+            v[1] = sf_pack2(acc[i][tt][2], acc[i][tt][3]);
+            sf_handoff_store(reinterpret_cast<sf_u32x2*>(p + unit * 16), v);
+          }
+        }
+      }
+    }
+  }
+};
+
+template <int NT>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void head_tile_kernel(const uint16_t* __restrict__ X, int Mo, HeadRows hr,
+                      const uint16_t* __restrict__ W, int K, int cols, uint16_t* __restrict__ out,
+                      long long ldo) {
+  __shared__ sf_u32x4 ring[kLdsBudget / 16];
+  const TileGemm g{X, K, W, nullptr, K, cols / 16};
+  auto in_row = [&](int r) { return head_in_row(r, hr); };
+  const HeadTileStore st{hr, out, ldo, cols / 16};
+  if (tile_nmt(Mo) == 3)
+    tile_items<false, 3, NT>(g, Mo, 1, ring, in_row, st);
+  else
+    tile_items<false, 4, NT>(g, Mo, 1, ring, in_row, st);
+}
+
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 }  // namespace
@@ -285,6 +337,33 @@ void head_launch(const uint16_t* x, int Mo, const HeadRows& hr, const uint16_t* 
   }
 }
 
+// Rows the tile GEMM takes.  Measured against passes of 256 rows, us (V = 152064 at
+// D = 3584, 151936 at 1536, 131072 at 5120):
+//   rows        136        160        192        256        320        512        640        1024
+//   D = 1536  127/132    136/136    153/139    175/151    245/278    330/310    407/445    597/623
+//   D = 3584  281/323    254/291    261/284    310/290    442/555    570/601    740/873   1030/1209
+//   D = 5120  269/312    274/307    287/308    351/317    480/615    645/637    870/960   1272/1290
+// (tiles/passes): tiles lose where a pass is full (its larger fixed cost per tile shows
+// the more the shorter K is) and win where rows are missing from it or blocks are many.
+bool head_tiles(int Mo, int D) {
+  const int nb = tile_blocks(Mo);
+  return nb >= 3 || (tile_nmt(Mo) == 3 && (nb == 2 || D >= 2048));
+}
+
+void head_tile_launch(const uint16_t* x, int Mo, const HeadRows& hr, const uint16_t* w, int D,
+                      int V, uint16_t* logits, long long ld_out, hipStream_t st) {
+  constexpr int kCUs = 256;
+  const int nb = tile_blocks(Mo);
+  // columns of the whole rounds of 256-column tiles, one (tile, row block) per CU
+  const int cols = (int)((long long)(V / 256) * nb / kCUs) * kCUs / nb * 256;
+  if (cols)
+    hipLaunchKernelGGL(head_tile_kernel<8>, dim3(kCUs), dim3(512), 0, st, x, Mo, hr, w, D, cols,
+                       logits, ld_out);
+  if (cols < V)
+    hipLaunchKernelGGL(head_tile_kernel<4>, dim3(kCUs), dim3(512), 0, st, x, Mo, hr,
+                       w + (size_t)cols * D, D, V - cols, logits + cols, ld_out);
+}
+
 }  // namespace
 
 extern "C" int sf_head_logits_rows(const uint16_t* x, int M, const uint16_t* w, int D, int V,
@@ -301,6 +380,8 @@ extern "C" int sf_head_logits_rows(const uint16_t* x, int M, const uint16_t* w, 
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (Mo <= HeadMain128::kRows)
     head_launch<HeadMain128, HeadTail128>(x, Mo, hr, w, D, V, logits, ld_out, st);
+  else if (head_tiles(Mo, D))
+    head_tile_launch(x, Mo, hr, w, D, V, logits, ld_out, st);
   else
     head_launch<HeadMain, HeadTail>(x, Mo, hr, w, D, V, logits, ld_out, st);
   return sf_launch_status();
