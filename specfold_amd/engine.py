@@ -572,6 +572,8 @@ class FoldedVerifyEngine:
             n = blk.shape[1]
             qs = None if q_scale is None else q_scale(cache.length, n)
             self.append_blocks(blk, cache, block, causal=causal, q_scale=qs, out=logits[s:s + n])
+        # as after a forward of the last block alone
+        self.last_hidden = self.last_hidden[(n - 1) // block * block:]
         return logits[:, :self.V].contiguous().view(1, L, self.V)
 
     @torch.no_grad()
@@ -921,7 +923,7 @@ class FoldedVerifyEngine:
     def profile_launchers(self, li: int = -1, shared: Optional[dict] = None):
         """No-argument callables that re-launch each HIP entry point of layer
         ``li`` (its weights, its slice of the cache) on the buffers resident from
-        the last forward (for timing).  The gate runs on the last layer's output
+        the last forward (for timing; append_blocks' buffers are its own).  The gate runs on the last layer's output
         hidden states, so call it last: it rewrites rows/count/src for the other
         launchers.  ``shared`` (a dict) lets the launchers of several layers
         share their scratch outputs."""

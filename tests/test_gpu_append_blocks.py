@@ -83,10 +83,14 @@ def test_prompt_matches_blocks(family, lengths):
     for n in lengths:
         t = torch.randint(0, 900, (1, n), generator=g)
         got = run(t, whole).logits
+        hidden = ex.engine.last_hidden.clone()
         ref = torch.cat([run(t[:, s:s + 32], parts).logits for s in range(0, n, 32)], dim=1)
         assert got.shape == ref.shape and got.is_contiguous()
         rel = (got.double() - ref.double()).norm() / ref.double().norm()
         assert rel < 1.6e-2, rel
+        last = ex.engine.last_hidden       # the last block's
+        assert hidden.shape == last.shape
+        assert (hidden.double() - last.double()).norm() / last.double().norm() < 1.6e-2
     assert whole.length == parts.length == int(whole.length_dev) == sum(lengths)
     for li in range(3):
         for a, b in zip(whole[li], parts[li]):
