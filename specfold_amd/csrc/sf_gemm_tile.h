@@ -336,6 +336,14 @@ SF_DEV void tile_items(const TileGemm& g, int M, int n_ranges, sf_u32x4* ring, c
   }
 }
 
+// The stores below are plain, not the hand-off stores of the few-row kernels: a store
+// instruction covers 64 (fp32) or 32 bytes (bf16) of a row, which the non-temporal hint
+// sends on as they are, part of a line each, while plain ones meet in L2 and leave as
+// whole lines.  From 129 rows on that outweighs the dirty lines the next kernel's
+// weight stream finds (non-temporal -> plain, us: QKV + o_proj of 144 of 640 rows
+// at 4096 78.5 -> 76.8; MLP of 256 rows at 5120 x 17408 187.5 -> 185.0; with the head's,
+// prefill of 2048 tokens, 4 layers at 7B widths 7408 -> 6867).
+
 // fp32 sums of K range s to part[(s * mcap + m) * N + c]
 struct TilePartStore {
   float* part;
@@ -354,7 +362,7 @@ struct TilePartStore {
         for (int tt = 0; tt < NT; ++tt) {
           const int unit = u0 + cg * NT + tt;
           if (unit * 16 < N)
-            sf_handoff_store(reinterpret_cast<sf_f32x4*>(p + unit * 16), acc[i][tt]);
+            *reinterpret_cast<sf_f32x4*>(p + unit * 16) = acc[i][tt];
         }
       }
     }
@@ -409,7 +417,7 @@ struct TileSiluStore {
         sf_u32x2 v;
         v[0] = sf_pack2(r[0], r[1]);
         v[1] = sf_pack2(r[2], r[3]);
-        sf_handoff_store(reinterpret_cast<sf_u32x2*>(p + (u0 + tt) * 16), v);
+        *reinterpret_cast<sf_u32x2*>(p + (u0 + tt) * 16) = v;
       }
     }
   }

@@ -287,7 +287,7 @@ struct HeadTileStore {
             sf_u32x2 v;
             v[0] = sf_pack2(acc[i][tt][0], acc[i][tt][1]);
             v[1] = sf_pack2(acc[i][tt][2], acc[i][tt][3]);
-            sf_handoff_store(reinterpret_cast<sf_u32x2*>(p + unit * 16), v);
+            *reinterpret_cast<sf_u32x2*>(p + unit * 16) = v;
           }
         }
       }
