@@ -264,12 +264,16 @@ void head_kernel(const uint16_t* __restrict__ X, int Mo, int m0, HeadRows hr,
 // above bit for bit (K ascending in one accumulator).  Its cost follows the row blocks
 // (192 or 256 rows each, several in one launch), where the kernel above pays a whole
 // pass over the weights per 256 rows whatever they hold.
-//
+// Stores: non-temporal up to 256 rows (a verify step), plain above (prompts).  32 bytes of
+// a row a store, plain ones leave L2 as whole lines (1024 rows of 152064: 1030 -> 958 us),
+// but the next forward's weight streams find them there: 256 rows on plain tile stores
+// took 287 us against a pass's 296, and the 8-layer verify step 1568 against 1557.
 struct HeadTileStore {
   HeadRows hr;
   uint16_t* out;
   long long ldo;
   int units;
+  bool stream;   // non-temporal stores
   template <int NMT, int NT>
   SF_DEV void operator()(int m0, int mrows, int, int u0, int rgrp, int cg,
                          const sf_f32x4 (&acc)[NMT][NT]) const {
@@ -287,7 +291,10 @@ struct HeadTileStore {
             sf_u32x2 v;
             v[0] = sf_pack2(acc[i][tt][0], acc[i][tt][1]);
             v[1] = sf_pack2(acc[i][tt][2], acc[i][tt][3]);
-            *reinterpret_cast<sf_u32x2*>(p + unit * 16) = v;
+            if (stream)
+              sf_handoff_store(reinterpret_cast<sf_u32x2*>(p + unit * 16), v);
+            else
+              *reinterpret_cast<sf_u32x2*>(p + unit * 16) = v;
           }
         }
       }
@@ -303,7 +310,7 @@ void head_tile_kernel(const uint16_t* __restrict__ X, int Mo, HeadRows hr,
   __shared__ sf_u32x4 ring[kLdsBudget / 16];
   const TileGemm g{X, K, W, nullptr, K, cols / 16};
   auto in_row = [&](int r) { return head_in_row(r, hr); };
-  const HeadTileStore st{hr, out, ldo, cols / 16};
+  const HeadTileStore st{hr, out, ldo, cols / 16, Mo <= 256};
   if (tile_nmt(Mo) == 3)
     tile_items<false, 3, NT>(g, Mo, 1, ring, in_row, st);
   else
@@ -337,17 +344,18 @@ void head_launch(const uint16_t* x, int Mo, const HeadRows& hr, const uint16_t* 
   }
 }
 
-// Rows the tile GEMM takes.  Measured against passes of 256 rows, us (V = 152064 at
-// D = 3584, 151936 at 1536, 131072 at 5120):
+// Rows the tile GEMM takes.  Measured against passes of 256 rows, us, non-temporal
+// stores up to 256 rows and plain ones above (V = 152064 at D = 3584, 151936 at 1536,
+// 131072 at 5120):
 //   rows        136        160        192        256        320        512        640        1024
-//   D = 1536  127/132    136/136    153/139    175/151    245/278    330/310    407/445    597/623
-//   D = 3584  281/323    254/291    261/284    310/290    442/555    570/601    740/873   1030/1209
-//   D = 5120  269/312    274/307    287/308    351/317    480/615    645/637    870/960   1272/1290
-// (tiles/passes): tiles lose where a pass is full (its larger fixed cost per tile shows
-// the more the shorter K is) and win where rows are missing from it or blocks are many.
+//   D = 1536  127/132    136/136    153/139    175/151    213/284    262/314    354/450    471/628
+//   D = 3584  281/323    254/291    261/284    310/290    435/576    525/618    723/894    958/1233
+//   D = 5120  269/312    274/307    287/308    351/317    480/654    594/679    857/997   1145/1357
+// (tiles/passes): tiles lose where one pass is full and win where rows are missing from it
+// or blocks are many (385 to 512 rows, two full passes, since the plain stores).
 bool head_tiles(int Mo, int D) {
   const int nb = tile_blocks(Mo);
-  return nb >= 3 || (tile_nmt(Mo) == 3 && (nb == 2 || D >= 2048));
+  return nb >= 2 || (tile_nmt(Mo) == 3 && D >= 2048);
 }
 
 void head_tile_launch(const uint16_t* x, int Mo, const HeadRows& hr, const uint16_t* w, int D,
