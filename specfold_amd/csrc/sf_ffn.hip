@@ -426,9 +426,10 @@ namespace {
 // More than 256 rows: the tile GEMM over the all-rows GEMM's K ranges (the same sums, bit
 // for bit), one launch for every row instead of one per 256, each with its own ring
 // fill and drain.  o_proj + residual + norm, 320 / 640 / 1024 rows: 33.8 / 51.4 / 71.1 ->
-// 26.7 / 43.7 / 56.4 us at 3584, 54.2 / 81.2 / 111.8 -> 41.0 / 63.4 / 81.1 at 5120.  (Both with
-// non-temporal stores; with the plain ones since, 640 rows at 4096 take 1.7 us less.)  At 129 to 256 rows
-// (one launch either way) the all-rows GEMM's narrower tiles are 1-10 % faster.
+// 26.7 / 43.7 / 56.4 us at 3584, 54.2 / 81.2 / 111.8 -> 41.0 / 63.4 / 81.1 at 5120 (with
+// non-temporal stores; the plain ones since take another 1.7 us off a QKV of 144 rows
+// with the o_proj of 640 at 4096).  At 129 to 256 rows (one launch either way) the
+// all-rows GEMM's narrower tiles are 1-10 % faster.
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void o_proj_tile_kernel(const uint16_t* __restrict__ A, int M, const uint16_t* __restrict__ W,
                         int K, int N, TilePlans tp, float* __restrict__ part) {
