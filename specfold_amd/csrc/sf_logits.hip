@@ -398,15 +398,28 @@ __global__ __launch_bounds__(kFinishThreads) void sf_logit_finish_kernel(
   float incl_p, tot_p;
   const float excl_p = block_scan<kFinishThreads>(part_p, s_v, incl_p, tot_p);
   if (tid == 0) s_cutf[1] = z;  // the nucleus mass when nothing is cut
-  __syncthreads();
   // The reference drops sorted token i >= 1 when bf16(cumsum_{j<i} p_j) > top_p:
   // the kept tokens run up to and including the first one whose cumulative
-  // probability crosses.  Exactly one stretch holds the crossing (monotone sums).
+  // probability crosses.  A thread's inclusive sum is the next one's exclusive sum,
+  // so the first whose inclusive sum crosses holds the crossing.  Others may pass the
+  // same test after it, and the first may be a stretch without tokens: the scan adds a
+  // thread's 64 predecessors in an order of its own, so where the mass ends within an
+  // ulp of a rounding boundary the sums of empty stretches lie on both sides of it.
+  // An empty one cuts at its start: the tokens before it are kept.
   auto crosses = [&](float cum) { return sf_rbf(cum) > top_p; };
-  if (!crosses(excl_p) && crosses(incl_p)) {
-    // the walk down the stretch to the first key whose mass crosses, in two halves
-    // of 32 counts, each read in one round of loads (count of key kb - j in
-    // cnt[j - 32 * half])
+  {
+    const unsigned long long bal = __ballot(!crosses(excl_p) && crosses(incl_p));
+    if ((tid & 63) == 0)
+      s_n[tid >> 6] = bal ? tid + __popcll((bal & (~bal + 1ull)) - 1ull) : kFinishThreads;
+  }
+  __syncthreads();
+  int first = kFinishThreads;
+#pragma unroll
+  for (int w = 0; w < kFinishThreads / 64; ++w) first = min(first, s_n[w]);
+  if (tid == first) {
+    // the walk down the stretch to the first key whose mass crosses, from LDS, or from
+    // memory in two halves of 32 counts, each read in one round of loads (count of key
+    // kb - j in cnt[j - 32 * half])
     float cp = excl_p, ce = excl_e;
     bool found = false;
     uint32_t cx = 0;
@@ -422,7 +435,7 @@ __global__ __launch_bounds__(kFinishThreads) void sf_logit_finish_kernel(
         ce += (float)c * e;
       }
     };
-    if (in_lds) {
+    if (slot >= 0) {
       for (int j0 = 63; j0 >= 0 && !found; j0 -= 16) {   // 16 keys' reads in flight
         uint32_t c[16];
         float e[16], pj[16];
