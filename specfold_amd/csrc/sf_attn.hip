@@ -270,8 +270,27 @@ SF_DEV void prefix_item(const uint16_t* __restrict__ q_buf, const uint16_t* __re
           acc[qs][dt] = sf_mfma16x16x32(sf_as_bf16x8(vw), pb[qs][pp], acc[qs][dt]);
       }
   };
+  // OWN: a hidden key has weight 0, but 0 * inf is NaN.  Where the carried chunk (its
+  // keys of this wave from key kb on) holds keys that a query of the wave does not see
+  // and a V value that is not finite, add_pv gets zeros and the chunk is noted: its P.V
+  // follows key by key after the range, for the queries that see the key.  Only the
+  // chunks around the own keys are looked at (~100 VALU operations each).
+  const int lim_min = OWN ? __builtin_amdgcn_readfirstlane(lim[0]) : 0;   // limits ascend
+  uint32_t noted = 0;   // bit u: chunk c1 - 1 - u (a tile's limits span 3 chunks at most)
+  auto hold_back = [&](int kb, sf_u32x2 (&vf)[16]) {
+    if (!OWN || kb + 32 <= lim_min) return;   // wave-uniform
+    uint32_t t = 0;   // bit 15 or 31: an exponent of all ones
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      t |= ((vf[i][0] & 0x7f807f80u) + 0x00800080u) | ((vf[i][1] & 0x7f807f80u) + 0x00800080u);
+    if (__ballot((t & 0x80008000u) != 0) == 0) return;
+    if (kb < c1 * kChunk) noted |= 1u << (c1 - 1 - kb / kChunk);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) vf[i] = sf_u32x2{0u, 0u};
+  };
 
-  // chunk c in the slot at `base`; the carried chunk's slot at `vbase`
+  // chunk c in the slot at `base`; the carried chunk's slot at `vbase`, its keys of this
+  // wave from key vkey on
   // a rescale of acc decided by a step, applied at the start of the next (after the
   // P.V that step added, before the one the next adds)
   bool resc_prev = false;
@@ -285,7 +304,7 @@ SF_DEV void prefix_item(const uint16_t* __restrict__ q_buf, const uint16_t* __re
     }
   };
 
-  auto step = [&](int c, sf_lds_off base, sf_lds_off vbase) {
+  auto step = [&](int c, sf_lds_off base, sf_lds_off vbase, int vkey) {
     rescale();
     sf_u32x4 kf[8];   // [t * 4 + ds]
 #pragma unroll
@@ -371,6 +390,7 @@ SF_DEV void prefix_item(const uint16_t* __restrict__ q_buf, const uint16_t* __re
 #pragma unroll
     for (int qs = 0; qs < 2; ++qs) m_use[qs] = m_ref[qs] == -INFINITY ? 0.f : m_ref[qs];
     sf_lds_reads_done(vf);
+    hold_back(vkey, vf);
     add_pv(vf);
     float lsum[2] = {0.f, 0.f};
 #pragma unroll
@@ -416,17 +436,75 @@ SF_DEV void prefix_item(const uint16_t* __restrict__ q_buf, const uint16_t* __re
     // (the first step's zero P parts take chunk 0's own V^T: landed, finite values,
     // where the carried slot would hold stale LDS bytes, possibly NaN patterns)
     const sf_lds_off cur = sf_lds_addr(ring + (k % kRing) * kSlotBytes);
-    step(c0 + k, cur, k == 0 ? cur : sf_lds_addr(ring + ((k + kRing - 1) % kRing) * kSlotBytes));
+    // (its keys: past every limit, so zeros meet no value that is not finite)
+    step(c0 + k, cur, k == 0 ? cur : sf_lds_addr(ring + ((k + kRing - 1) % kRing) * kSlotBytes),
+         (k == 0 ? kMaxChunks : c0 + k - 1) * kChunk + 32 * kh);
   }
   {  // the last chunk's P.V
     rescale();
     sf_u32x2 vf[16];
     read_vt(sf_lds_addr(ring + ((nck + kRing - 1) % kRing) * kSlotBytes), vf);
     sf_lds_reads_done(vf);
+    hold_back((c1 - 1) * kChunk + 32 * kh, vf);
     add_pv(vf);
   }
   // drain the clamped re-issues past the range end before the ring is reused
   sf_wait_vm_barrier<0>();
+
+  // ---- OWN: the P.V of the chunks held back, a key at a time -------------------------
+  if constexpr (OWN) {
+    // (the query rows again: qf kept to here would spill)
+    long long qat[2];
+#pragma unroll
+    for (int qs = 0; qs < 2; ++qs) {
+      const int qc = min(qt * kQT + qg * 32 + qs * 16 + ql, nq - 1);
+      const int m = qc / G;
+      qat[qs] = ((long long)m * H + h * G + (qc - m * G)) * kHD + grp * 8;
+    }
+#pragma unroll 1
+    for (int u = 0; noted >> u; ++u) {   // wave-uniform
+      if (!(noted >> u & 1u)) continue;
+      const int kb = (c1 - 1 - u) * kChunk + 32 * kh;
+#pragma unroll 1
+      for (int key = kb; key < min(kb + 32, P); ++key) {
+        long long at = head_off + (long long)key * kHD;
+        if (page_table)
+          at = head_off + (long long)s_pg[(key >> 4) - 4 * c0] * page_stride +
+               (long long)(key & (page_size - 1)) * kHD;
+        float dot[2] = {0.f, 0.f};
+#pragma unroll
+        for (int ds = 0; ds < 4; ++ds) {
+          float kv[8], qv[8];
+          sf_unpack8(*reinterpret_cast<const sf_u32x4*>(pk + at + ds * 32 + grp * 8), kv);
+#pragma unroll
+          for (int qs = 0; qs < 2; ++qs) {
+            sf_unpack8(*reinterpret_cast<const sf_u32x4*>(q_buf + qat[qs] + ds * 32), qv);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) dot[qs] = fmaf(kv[i], qv[i], dot[qs]);
+          }
+        }
+        float p[2];
+#pragma unroll
+        for (int qs = 0; qs < 2; ++qs) {
+          dot[qs] += __shfl_xor(dot[qs], 16, 64);
+          dot[qs] += __shfl_xor(dot[qs], 32, 64);
+          p[qs] = __builtin_amdgcn_exp2f(
+              fmaf(dot[qs], scale_log2, m_ref[qs] == -INFINITY ? 0.f : -m_ref[qs]));
+        }
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt) {
+          const sf_u32x2 w = *reinterpret_cast<const sf_u32x2*>(pv + at + dt * 16 + grp * 4);
+          const float v[4] = {__uint_as_float(w[0] << 16), __uint_as_float(w[0] & 0xffff0000u),
+                              __uint_as_float(w[1] << 16), __uint_as_float(w[1] & 0xffff0000u)};
+#pragma unroll
+          for (int qs = 0; qs < 2; ++qs)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              acc[qs][dt][i] = key < lim[qs] ? fmaf(p[qs], v[i], acc[qs][dt][i]) : acc[qs][dt][i];
+        }
+      }
+    }
+  }
 
   // ---- combine the two key halves of each query, write the partial -----------------
   // the query's maximum and l over its four lane groups
