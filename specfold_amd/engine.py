@@ -573,7 +573,10 @@ class FoldedVerifyEngine:
             qs = None if q_scale is None else q_scale(cache.length, n)
             self.append_blocks(blk, cache, block, causal=causal, q_scale=qs, out=logits[s:s + n])
         # as after a forward of the last block alone
-        self.last_hidden = self.last_hidden[(n - 1) // block * block:]
+        last = (n - 1) // block * block
+        self.last_hidden = self.last_hidden[last:]
+        self._last = dict(prompt=blk[:, last:], cache=cache, causal=causal,
+                          q_scale=None if qs is None else qs.reshape(-1)[last:])
         return logits[:, :self.V].contiguous().view(1, L, self.V)
 
     @torch.no_grad()
@@ -920,13 +923,32 @@ class FoldedVerifyEngine:
         return out
 
     # ------------------------------------------------------------------------
+    def _prompt_step(self, blk: torch.Tensor, cache: PagedKVCache, causal: bool,
+                     q_scale: Optional[torch.Tensor]) -> None:
+        """The last block of an append_prompt run as a step of its own over the tokens in
+        front of it, not appended: fills the step buffers that profile_launchers
+        re-launches on (append_blocks has its own)."""
+        saved = self.last_hidden, self.use_graphs, self.gate_mode
+        back = min(blk.shape[1], cache.length)
+        cache.advance(-back)
+        self.use_graphs, self.gate_mode = False, _lib.SF_GATE_ALL
+        try:
+            self.forward(blk, cache, delta=0.0, compute_logits=False, q_scale=q_scale,
+                         causal=causal)
+        finally:
+            cache.advance(back)
+            self.last_hidden, self.use_graphs, self.gate_mode = saved
+
     def profile_launchers(self, li: int = -1, shared: Optional[dict] = None):
         """No-argument callables that re-launch each HIP entry point of layer
         ``li`` (its weights, its slice of the cache) on the buffers resident from
-        the last forward (for timing; append_blocks' buffers are its own).  The gate runs on the last layer's output
-        hidden states, so call it last: it rewrites rows/count/src for the other
-        launchers.  ``shared`` (a dict) lets the launchers of several layers
-        share their scratch outputs."""
+        the last forward (for timing; after a prompt, its last block's step).  The gate
+        runs on the last layer's output hidden states, so call it last: it rewrites
+        rows/count/src for the other launchers.  ``shared`` (a dict) lets the launchers
+        of several layers share their scratch outputs."""
+        if "prompt" in self._last:
+            p = self._last
+            self._prompt_step(p["prompt"], p["cache"], p["causal"], p["q_scale"])
         st = self._last
         B1, N, bucket, cache = st["B1"], st["N"], st["bucket"], st["cache"]
         BN = B1 * N

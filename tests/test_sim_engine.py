@@ -13,6 +13,7 @@ import pytest
 import torch
 
 from oracle.folded_reference import StepTrace, folded_verify_step, llama4_q_scale
+from specfold_amd import _lib
 from specfold_amd.engine import FoldedVerifyEngine
 from specfold_amd.kv_cache import PagedKVCache
 from tests.helpers import (SHAPE_G2, SHAPE_G7, SHAPE_N4, err_stats, make_case, make_nld_case,
@@ -271,3 +272,30 @@ def test_batched_padding_at_delta_zero(sim):
         assert torch.equal(a, b)
     real = [sum(c) for c in zip(*counts)]
     assert all(b >= r for b, r in zip(st.counts, real)) and st.counts[0] == real[0]
+
+
+def test_profile_launchers_after_a_prompt(sim):
+    """After a cache-filling forward of several blocks alone, profile_launchers has its
+    last block's step to re-launch: the buffers that a forward of that block leaves, and
+    neither the cache nor the last hidden state changes."""
+    shape = SHAPE_G2
+    case = make_case(shape, 1, P=40)
+    cache, same = _paged(case.kv), _paged(case.kv)
+    tokens = torch.randint(0, shape.vocab - 1, (1, 72), generator=torch.Generator().manual_seed(3))
+    eng, ref = SimEngine(case.model_cpu), SimEngine(case.model_cpu)
+    ref.use_graphs = False
+    ref.gate_mode = _lib.SF_GATE_ALL
+    eng.append_prompt(tokens, cache, 32)
+    for s in (0, 32, 64):
+        ref.forward(tokens[:, s:s + 32], same, delta=0.0, append=True)
+    before = [t.clone() for t in (cache.k_pages, cache.v_pages, eng.last_hidden)]
+    (launch, info), (_, want) = eng.profile_launchers(), ref.profile_launchers()
+    assert set(launch) >= {"qkv", "attn", "o_proj", "gate_up", "down", "lm_head", "gate"}
+    assert info["prefix"] == want["prefix"] == cache.length == int(cache.length_dev) == 112
+    assert int(info["count"]) == int(want["count"]) == 8
+    a, b = info["buf"].final.float(), want["buf"].final.float()
+    # two bf16 forwards whose attention sums in another order
+    assert a.shape == b.shape and (a - b).norm() <= 1.6e-2 * b.norm()
+    assert all(torch.equal(x, y) for x, y in
+               zip(before, (cache.k_pages, cache.v_pages, eng.last_hidden)))
+    assert eng.use_graphs and eng.gate_mode == _lib.SF_GATE_MODEL_DTYPE
