@@ -292,7 +292,7 @@ __global__ __launch_bounds__(256) void down_fixup_kernel(const float* __restrict
   const int M = min(*count_p, mcap);
   const int nsl = tile_last(t, plan) - tile_first(t, plan) + 1;
   // (the tile GEMM leaves single slots to this kernel too)
-  if (nsl == 1 && !(M > kTileRows && tp.nt)) return;
+  if (nsl == 1 && !tile_takes(M, tp)) return;
   const int m = blockIdx.y * kFixRows + (threadIdx.x >> 5);
   if (m >= M) return;
   const size_t stride = (size_t)mcap * N;

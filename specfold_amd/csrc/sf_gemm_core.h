@@ -333,9 +333,9 @@ void gemm_sk_kernel(const uint16_t* __restrict__ A, const int32_t* __restrict__ 
     M = count_p ? sf_imin(*count_p, mcap) : m_static;
   }
   if constexpr (TILE) {
-    // workgroup-uniform: more rows than a pass below holds (and a plan the tile GEMM
-    // computes with the same sums: tp.nt = 0 otherwise)
-    if (M > kTileRows && tp.nt) {
+    // workgroup-uniform: more rows than a pass below holds, and a plan for them that the
+    // tile GEMM computes with the same sums
+    if (tile_takes(M, tp)) {
       const TileGemm tg{A, lda, W0, W1, K, N / 16};
       auto in_row = [&](int r) { return GATED ? s_grows[r] : (a_rows ? a_rows[r] : r); };
       if constexpr (MODE == kSilu) {
@@ -358,7 +358,7 @@ void gemm_sk_kernel(const uint16_t* __restrict__ A, const int32_t* __restrict__ 
   const size_t stride = (size_t)mcap * N;
   const int g = blockIdx.x;
   const int u_end = plan_range_end(g, plan);
-  // rows beyond MB (a launch whose mcap exceeds 256) take further passes
+  // rows beyond MB (128 at most; more that the tile GEMM does not take) in further passes
   for (int m0 = 0; m0 < M; m0 += MB) {
   const int mrows = sf_imin(MB, M - m0);
   const int nmt = (mrows + 15) >> 4;
@@ -481,7 +481,8 @@ void gemm_sk_kernel(const uint16_t* __restrict__ A, const int32_t* __restrict__ 
 
 // The kernel for a launch of at most mcap rows: 64 rows, 128 rows, or 128 rows with
 // the tile GEMM for device-side counts above that (one pass over the weights for
-// every 256 rows, where the streaming core would take one per 128).
+// every 256 rows, where the streaming core takes one per 128; rows that tile_takes
+// leaves take those passes in it, as fast as in the 128-row kernel).
 template <int WN, int MODE, bool GATED = false>
 inline void launch_sk(const Plan& p, const TilePlans& tp, const uint16_t* A, const int32_t* a_rows,
                       int lda, const int32_t* count_p, int m_static, int mcap, const uint16_t* W0,

@@ -279,9 +279,11 @@ SF_IDX int tile_nmt(int M) {
 }
 struct TilePlans {
   int ks = 1;        // K ranges
-  unsigned nt = 0;   // byte tile_blocks(M) - 1: NT
+  unsigned nt = 0;   // byte tile_blocks(M) - 1: NT, or 0: such rows stay on the streaming core
 };
 SF_IDX int tile_nt(int M, const TilePlans& p) { return (p.nt >> (8 * (tile_blocks(M) - 1))) & 255; }
+// Whether the tile GEMM computes M rows.
+SF_IDX bool tile_takes(int M, const TilePlans& p) { return M > kTileRows && tile_nt(M, p) != 0; }
 // Cycles of a workgroup per 32-wide K chunk: the LDS operand reads of 8 waves
 // (128 B a cycle) with the copies' writes, or two waves' MFMAs per SIMD.
 inline long long tile_chunk_cycles(int nmt, int nt) {
@@ -294,6 +296,16 @@ inline long long tile_chunk_cycles(int nmt, int nt) {
 // of whole rounds of the grid (never below the weight stream, ~2000 bytes a cycle)
 // and a fixed cost per item.  The K ranges are those of the streaming core's plan
 // (a whole K, or its split plan), so a row's sums are the same for every row count.
+// Short ranges are all ring fill and partial sums, and the streaming core's narrower
+// pieces overlap those of several passes: with K cut up, the tile GEMM takes rows from
+// 3 / 2 / 2 / 1 stages in a range on, on average, for 1 / 2 / 3 / 4 row blocks.  Measured,
+// streaming -> tile, us, ranges of 1.0 to 1.4 / 2 / 2.75 / 3.3 to 3.6 stages:
+//   256 rows: down 1024 x 1408 18.8 -> 21.9 / QKV 2048 x 1536 22.2 -> 25.4 / down
+//     2048 x 2816 22.5 -> 25.9 / down 768 x 8960 31.2 -> 24.3, 1536 x 4864 29.6 -> 24.5
+//   257-320: down 2048 x 1408 23.0 -> 26.0 / QKV 29.4 -> 29.5 (512: 38.0 -> 34.2) / 28.8 ->
+//     27.3 / 37.1 -> 29.1, 35.1 -> 28.6
+//   640: down 1024 x 1408 35.6 -> 37.3 / QKV 46.0 -> 45.9 / 48.3 -> 47.7 / 63.3 -> 51.1
+//   1024: down 1024 x 1408 53.1 -> 45.5 / QKV 72.8 -> 57.8 / 74.5 -> 60.0 / 99.0 -> 62.0
 inline TilePlans make_tile_plans(int units, int K, bool silu, int ks) {
   TilePlans p;
   p.ks = ks;
@@ -314,6 +326,8 @@ inline TilePlans make_tile_plans(int units, int K, bool silu, int ks) {
         best_nt = (unsigned)nt;
       }
     }
+    const int least = b == 1 ? 3 : (b <= 3 ? 2 : 1);
+    if (ks > 1 && K / 64 < least * ks) best_nt = 0;
     p.nt |= best_nt << (8 * (b - 1));
   }
   return p;

@@ -18,6 +18,8 @@ def sim(tmp_path_factory):
 @pytest.mark.parametrize("case", [
     (128, 256, 270, 288, 30, 21),   # D, I, count, bucket, M, seed: blocks of 192 rows
     (128, 384, 250, 256, 30, 22),   # one block of 256
+    (128, 768, 270, 288, 30, 23),   # 12 stages of down in 3 ranges: its tiles' partial sums
+    (128, 768, 250, 256, 30, 24),
 ], ids=lambda c: "D%d_I%d_count%d_bucket%d_M%d" % c[:5])
 def test_tile_gemm(sim, case):
     r = subprocess.run([str(sim), *map(str, case)], capture_output=True, text=True, timeout=600)
