@@ -21,47 +21,6 @@
 
 namespace sfg {
 
-template <int NMT, int NT>
-struct TileShape {
-  static constexpr int kRB = 64 * NMT;            // rows of a block
-  static constexpr int kAW = 8 * NMT * 64;        // 16-byte words of A per stage (64 K)
-  static constexpr int kNW = 2 * NT;              // weight copies (1 KB) per chunk (32 K)
-  static constexpr int kWW = kNW * 64;            // words of weights per chunk
-  // A stages: 3 (copied two stages ahead) where four weight chunks fit beside them
-  static constexpr int kRA = (kLdsBudget / 16 - 3 * kAW) / kWW >= 4 ? 3 : 2;
-  static constexpr int kRWmax = (kLdsBudget / 16 - kRA * kAW) / kWW;
-  static constexpr int kRW = kRWmax < 6 ? kRWmax : 6;   // weight chunks
-  static constexpr int kWords = kRA * kAW + kRW * kWW;
-  static constexpr int kCW = (kNW + 7) / 8;       // weight copies per wave (the last: waves
-  static constexpr int kRem = kNW % 8;            // below kRem, if it is not 0)
-  static_assert(kRW >= 3 && kRW >= 2 * kRA - 2, "ring depths");
-  // Copies go out in windows, window c from chunk c's barrier to chunk c + 1's: the A
-  // rows of stage (c - 1)/2 + kRA when c is odd, then the weights of chunk c - 1 + kRW.
-  // Copies of a wave (w weight copies per chunk) in windows [a, b).
-  static constexpr int window_copies(int a, int b, int w) {
-    int n = 0;
-    for (int v = a; v < b; ++v) n += (v - 1 + kRW >= 0 ? w : 0) + ((v & 1) ? NMT : 0);
-    return n;
-  }
-  // Younger copies than those chunk c + 1 needs, at chunk c's barrier (c = 2 + k stands
-  // for every c of its parity once the windows are regular): its weights went out in
-  // window c + 2 - kRW, and when c is odd the A rows of its stage in c + 2 - 2 kRA.
-  static constexpr int in_flight(int k, int w) {
-    const int c = 2 * kRA + 2 * kRW + k;
-    const int nw = window_copies(c + 3 - kRW, c, w);
-    const int na = w + window_copies(c + 3 - 2 * kRA, c, w);
-    return k == 1 && na < nw ? na : nw;
-  }
-  // ... than those chunk 0 needs, after the prologue (windows below 0)
-  static constexpr int in_flight_first(int w) {
-    const int nw = window_copies(2 - kRW, 0, w);
-    const int na = (2 - 2 * kRA - 1 + kRW > 0 ? w : 0) + window_copies(2 - 2 * kRA, 0, w);
-    return na < nw ? na : nw;
-  }
-  // chunks before the end at which the windows stop being regular
-  static constexpr int kTail = 2 * kRA > kRW - 1 ? 2 * kRA : kRW - 1;
-};
-
 // At most N of this wave's vector-memory loads in flight, then the workgroup barrier.
 // Its LDS reads stay in flight (sf_wait_vm_barrier would wait for them).
 template <int N>
@@ -76,29 +35,6 @@ SF_DEV void tile_barrier() {
   sf_wait_vm_barrier<N>();
 #endif
 }
-// The order of a wave's LDS reads and how many of them may be in flight at each use.
-// The MFMAs of a chunk go in NT steps, step t those of weight tile t with the NMT A
-// tiles; D steps ahead of it the step's fragments are read: step t reads weight
-// fragment t + D of its chunk while t < NT - D, and from step NT - D on, fragment
-// j = t - (NT - D) of the NEXT chunk, the first NA0 of its A fragments in front of
-// j = 0 and the others in front of j = 1 (D = 1: all in front of j = 0).
-template <int NMT, int NT>
-struct TileSteps {
-  static constexpr int kD = NT >= 4 ? 3 : NT - 1;
-  static constexpr int kNA0 = kD == 1 ? NMT : (NMT + 1) / 2;
-  static constexpr int a_reads(int j) { return j == 0 ? kNA0 : j == 1 ? NMT - kNA0 : 0; }
-  static constexpr int reads(int t) { return t < NT - kD ? 1 : 1 + a_reads(t - (NT - kD)); }
-  // reads issued after the ones step t uses, its own step's reads included
-  static constexpr int later(int t) {
-    int n = 0;
-    for (int i = 1; i <= kD; ++i) n += reads((t - kD + i + NT) % NT);
-    // step 0 also takes the A fragments, the last of them in front of j = 1's weight
-    // fragment: of the reads after j = 0's, those A reads must have landed too
-    if (t == 0 && kD > 1) n -= a_reads(1);
-    return n;
-  }
-};
-
 // Fragments [I, E) of f, STEP bytes apart from LDS byte address a (that of fragment
 // 0), without waiting.
 template <int STEP, int I, int E, int N>

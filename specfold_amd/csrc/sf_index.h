@@ -48,22 +48,14 @@ SF_IDX P weight_lane_ptr(P W, int tile16, int K, int lane) {
 // A stage of the GEMM core is 64 K, two 32-wide MFMA chunks; chunk c of stage sc:
 SF_IDX int weight_chunk(int sc, int c) { return 2 * sc + c; }
 
-// A operand in LDS: per (chunk, m tile) a 1 KB tile of 16 rows x 64 bytes whose
-// four 16-byte units are XOR-swizzled (unit u of row r at position u ^ a_swz(r)).
-// Direct copy j of wave wv brings (chunk, m tile) q = a_copy(wv, j, NMT) = ch*NMT
-// + mt (waves with fewer real copies repeat the last one); its lane L writes word
-// L of the tile (row L/4, position L%4) with A unit a_copy_unit(L) of that row.
-// The MFMA reader lane l (row l%16, unit l/16) reads word a_read_word(l).
-SF_IDX int a_swz(int r) { return (r >> 1) & 3; }
+// A operand in LDS: per m tile 16 rows x 128 bytes (a stage's 64 K), brought by two
+// direct copies of 8 rows each, so that every copy takes whole 128-byte cache lines.
+// (Two copies that share a line stall the vector cache: the second hits a line whose
+// data is still on its way.)  Copy j of wave wv is a_copy(wv, j, NMT) of the 2·NMT (waves
+// with fewer real copies repeat the last one).  Word r*8 + (u ^ r%8) holds unit u of row
+// r: lane L of a copy brings unit a2_copy_unit(L) of row L/8; the MFMA reader lane l of
+// chunk k (unit 4k + l/16 of row l%16) reads word a2_read_word(l, k).
 SF_IDX int a_copy(int wv, int j, int NMT) { return sf_imin(wv + 8 * j, 2 * NMT - 1); }
-SF_IDX int a_copy_unit(int L) { return (L & 3) ^ a_swz(L >> 2); }
-SF_IDX int a_read_word(int l) { return (l & 15) * 4 + ((l >> 4) ^ a_swz(l & 15)); }
-// The same for a whole 64-K stage at once: 16 rows x 128 bytes, two copies of 8 rows
-// each, so every copy takes whole 128-byte cache lines.  (Two copies that share a
-// line stall the vector cache: the second hits a line whose data is still on its way.)
-// Word r*8 + (u ^ r%8) holds unit u of row r: lane L of a copy brings unit
-// a2_copy_unit(L) of row L/8; the fragment reader lane l of chunk k (unit 4k + l/16 of
-// row l%16) reads word a2_read_word(l, k).
 SF_IDX int a2_copy_unit(int L) { return (L & 7) ^ (L >> 3); }
 SF_IDX int a2_read_word(int l, int k) {
   return (l & 15) * 8 + ((4 * k + (l >> 4)) ^ (l & 7));
@@ -253,11 +245,9 @@ inline int rows_splits(int M, int N, int K, int ks_max) {
   const int rg = rows_rg(sf_imin(256, M));
   return make_rows_plan(rows_tiles<WN>(N, rg), rows_stages(K), ks_max).KS;
 }
-// Copy q of a stage (clamped to the last real copy): A tile (chunk q / MT, m tile
-// q % MT, in the tile layout of a_copy); weight block (tile q / CPS, chunk q % CPS).
+// Copy q of a stage (clamped to the last real copy): rows 8q .. +8 of A; weight block
+// (tile q / CPS, chunk q % CPS).
 SF_IDX int rows_a_copy(int q, int NA) { return sf_imin(q, NA - 1); }
-SF_IDX int rows_a_chunk(int q, int MT) { return q / MT; }
-SF_IDX int rows_a_mtile(int q, int MT) { return q % MT; }
 SF_IDX int rows_w_copy(int q, int NW) { return sf_imin(q, NW - 1); }
 SF_IDX int rows_w_tile(int q, int CPS) { return q / CPS; }
 SF_IDX int rows_w_chunk(int q, int CPS) { return q % CPS; }
@@ -277,6 +267,71 @@ SF_IDX int tile_nmt(int M) {
   const int nb = tile_blocks(M);
   return (M + nb - 1) / nb <= 192 ? 3 : 4;
 }
+// The ring of a workgroup tile of 64·NMT rows x 32·NT columns.
+template <int NMT, int NT>
+struct TileShape {
+  static constexpr int kRB = 64 * NMT;            // rows of a block
+  static constexpr int kAW = 8 * NMT * 64;        // 16-byte words of A per stage (64 K)
+  static constexpr int kNW = 2 * NT;              // weight copies (1 KB) per chunk (32 K)
+  static constexpr int kWW = kNW * 64;            // words of weights per chunk
+  // A stages: 3 (copied two stages ahead) where four weight chunks fit beside them
+  static constexpr int kRA = (kLdsBudget / 16 - 3 * kAW) / kWW >= 4 ? 3 : 2;
+  static constexpr int kRWmax = (kLdsBudget / 16 - kRA * kAW) / kWW;
+  static constexpr int kRW = kRWmax < 6 ? kRWmax : 6;   // weight chunks
+  static constexpr int kWords = kRA * kAW + kRW * kWW;
+  static constexpr int kCW = (kNW + 7) / 8;       // weight copies per wave (the last: waves
+  static constexpr int kRem = kNW % 8;            // below kRem, if it is not 0)
+  static_assert(kRW >= 3 && kRW >= 2 * kRA - 2, "ring depths");
+  // Copies go out in windows, window c from chunk c's barrier to chunk c + 1's: the A
+  // rows of stage (c - 1)/2 + kRA when c is odd, then the weights of chunk c - 1 + kRW.
+  // Copies of a wave (w weight copies per chunk) in windows [a, b).
+  static constexpr int window_copies(int a, int b, int w) {
+    int n = 0;
+    for (int v = a; v < b; ++v) n += (v - 1 + kRW >= 0 ? w : 0) + ((v & 1) ? NMT : 0);
+    return n;
+  }
+  // Younger copies than those chunk c + 1 needs, at chunk c's barrier (c = 2 + k stands
+  // for every c of its parity once the windows are regular): its weights went out in
+  // window c + 2 - kRW, and when c is odd the A rows of its stage in c + 2 - 2 kRA.
+  static constexpr int in_flight(int k, int w) {
+    const int c = 2 * kRA + 2 * kRW + k;
+    const int nw = window_copies(c + 3 - kRW, c, w);
+    const int na = w + window_copies(c + 3 - 2 * kRA, c, w);
+    return k == 1 && na < nw ? na : nw;
+  }
+  // ... than those chunk 0 needs, after the prologue (windows below 0)
+  static constexpr int in_flight_first(int w) {
+    const int nw = window_copies(2 - kRW, 0, w);
+    const int na = (2 - 2 * kRA - 1 + kRW > 0 ? w : 0) + window_copies(2 - 2 * kRA, 0, w);
+    return na < nw ? na : nw;
+  }
+  // chunks before the end at which the windows stop being regular
+  static constexpr int kTail = 2 * kRA > kRW - 1 ? 2 * kRA : kRW - 1;
+};
+
+// The order of a wave's LDS reads and how many of them may be in flight at each use.
+// The MFMAs of a chunk go in NT steps, step t those of weight tile t with the NMT A
+// tiles; D steps ahead of it the step's fragments are read: step t reads weight
+// fragment t + D of its chunk while t < NT - D, and from step NT - D on, fragment
+// j = t - (NT - D) of the NEXT chunk, the first NA0 of its A fragments in front of
+// j = 0 and the others in front of j = 1 (D = 1: all in front of j = 0).
+template <int NMT, int NT>
+struct TileSteps {
+  static constexpr int kD = NT >= 4 ? 3 : NT - 1;
+  static constexpr int kNA0 = kD == 1 ? NMT : (NMT + 1) / 2;
+  static constexpr int a_reads(int j) { return j == 0 ? kNA0 : j == 1 ? NMT - kNA0 : 0; }
+  static constexpr int reads(int t) { return t < NT - kD ? 1 : 1 + a_reads(t - (NT - kD)); }
+  // reads issued after the ones step t uses, its own step's reads included
+  static constexpr int later(int t) {
+    int n = 0;
+    for (int i = 1; i <= kD; ++i) n += reads((t - kD + i + NT) % NT);
+    // step 0 also takes the A fragments, the last of them in front of j = 1's weight
+    // fragment: of the reads after j = 0's, those A reads must have landed too
+    if (t == 0 && kD > 1) n -= a_reads(1);
+    return n;
+  }
+};
+
 struct TilePlans {
   int ks = 1;        // K ranges
   unsigned nt = 0;   // byte tile_blocks(M) - 1: NT, or 0: such rows stay on the streaming core

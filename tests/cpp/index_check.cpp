@@ -177,8 +177,9 @@ static void check_plans() {
                           {896, 1152, 4864, 151936}};
   for (const Shape& s : shapes) {
     for (int mcap : {1, 39, 64, 65, 128, 129, 256, 1024}) {
-      // QKV: 128-column tiles, 64-K stages, stream-K, partial slots [slots][bucket][n_qkv]
-      const sfg::Plan q = sfg::make_plan(s.nqkv / 128, s.D / 64);
+      // QKV: 128-column tiles, 64-K stages, each tile cut into whole K ranges of at least
+      // two stages, partial slots [slots][bucket][n_qkv]
+      const sfg::Plan q = sfg::make_plan_split(s.nqkv / 128, s.D / 64, 2);
       const int qs = walk_plan(q, false);
       const size_t need_q = (size_t)(qs + 1) * mcap * s.nqkv * sizeof(float);
       CHECK(f_qkv_ws(mcap, s.D, s.nqkv) >= need_q, "qkv workspace D=%d", s.D);
@@ -225,21 +226,21 @@ static void walk_rows_pass(const sfg::RowsPlan& p, int M, int m0, int mb, int N,
     if (s == 0) CHECK(s0 == 0, "first range");
     if (s == p.KS - 1) CHECK(s1 == p.S, "last range");
   }
-  // copies of one stage: each A tile (chunk, m tile) and weight block (tile, chunk)
+  // copies of one stage: each A copy (8 rows of 64 K) and weight block (tile, chunk)
   // at least once over the 8 waves (waves past the last copy repeat it)
   constexpr int CPS = St::kCPS;
   std::vector<int> acell(St::kNA, 0), wcell(St::kNW, 0);
+  CHECK(St::kNA * 8 == St::kMB, "A copies of the rows");
   for (int wv = 0; wv < 8; ++wv) {
     for (int j = 0; j < St::kDA; ++j) {
       const int cq = sfg::rows_a_copy(wv + 8 * j, St::kNA);
-      const int ch = sfg::rows_a_chunk(cq, St::kMT), mt = sfg::rows_a_mtile(cq, St::kMT);
-      CHECK(ch < CPS && mt < St::kMT, "a copy");
-      ++acell[ch * St::kMT + mt];
+      CHECK(cq >= 0 && cq < St::kNA, "a copy");
+      ++acell[cq];
       for (int L = 0; L < 64; ++L) {
-        const int r = sf_imin(mt * 16 + (L >> 2), mb - 1);
+        const int r = sf_imin(cq * 8 + (L >> 3), mb - 1);
         CHECK(r >= 0 && r < mb && m0 + r < M, "a row");
-        const size_t last = (size_t)(m0 + r) * K + (size_t)(p.S - 1) * St::kKS + ch * 32 +
-                            sfg::a_copy_unit(L) * 8 + 8;
+        const size_t last = (size_t)(m0 + r) * K + (size_t)(p.S - 1) * St::kKS +
+                            sfg::a2_copy_unit(L) * 8 + 8;
         CHECK(last <= (size_t)M * K, "a load");
       }
     }
@@ -266,7 +267,7 @@ static void walk_rows_pass(const sfg::RowsPlan& p, int M, int m0, int mb, int N,
     for (int lane = 0; lane < 64; ++lane)
       for (int c = 0; c < CPS; ++c) {
         for (int i = 0; i < 8; ++i) {
-          const int w = (c * St::kMT + rgrp * 8 + i) * 64 + sfg::a_read_word(lane);
+          const int w = (rgrp * 8 + i) * 128 + sfg::a2_read_word(lane, c);
           CHECK(w >= 0 && w < St::kA, "a read word %d", w);
         }
         for (int tt = 0; tt < WN; ++tt) {
@@ -380,9 +381,10 @@ static void check_columns(int N, int K) {
   }
 }
 
-// The A operand's LDS tiles: the copies of a stage cover every (chunk, m tile)
-// (extra copies only repeat the last), and the MFMA reader of every lane finds
-// the A unit its fragment needs.
+// The A operand's LDS tiles (16 rows x 64 K, 128 words): the copies of a stage, 8 rows
+// each, cover every tile's halves (extra copies only repeat the last) with rows of the
+// pass and whole 128-byte lines, and the MFMA reader of every lane and chunk finds the A
+// unit its fragment needs, the 8 lanes of an eighth of a wave on distinct bank groups.
 static void check_a_tiles() {
   for (int NMT : {1, 2, 3, 4, 5, 8, 16}) {
     const int DPW = (2 * NMT + 7) / 8;
@@ -393,29 +395,32 @@ static void check_a_tiles() {
         CHECK(q >= 0 && q < 2 * NMT, "copy %d out of range", q);
         ++got[q];
       }
-    for (int q = 0; q < 2 * NMT - 1; ++q) CHECK(got[q] == 1, "tile %d copied %d times", q, got[q]);
-    CHECK(got[2 * NMT - 1] >= 1, "last tile never copied");
+    for (int q = 0; q < 2 * NMT - 1; ++q) CHECK(got[q] == 1, "copy %d made %d times", q, got[q]);
+    CHECK(got[2 * NMT - 1] >= 1, "last copy never made");
   }
-  // word w of a tile holds unit a_copy_unit(w) of row w/4
-  int unit_at[64], row_at[64];
-  std::vector<int> seen(64, 0);
-  for (int L = 0; L < 64; ++L) {
-    unit_at[L] = sfg::a_copy_unit(L);
-    row_at[L] = L >> 2;
-    ++seen[row_at[L] * 4 + unit_at[L]];
-  }
-  for (int i = 0; i < 64; ++i) CHECK(seen[i] == 1, "(row, unit) %d stored %d times", i, seen[i]);
-  for (int l = 0; l < 64; ++l) {
-    const int w = sfg::a_read_word(l);
-    CHECK(w >= 0 && w < 64, "read word");
-    CHECK(row_at[w] == (l & 15) && unit_at[w] == (l >> 4), "lane %d reads the wrong unit", l);
-  }
-  // the 8 lanes of each quarter-wave read distinct 16-byte bank groups
-  for (int g = 0; g < 8; ++g) {
-    int mask = 0;
-    for (int l = 8 * g; l < 8 * g + 8; ++l) mask |= 1 << (sfg::a_read_word(l) & 7);
-    CHECK(mask == 0xff, "bank groups of lanes %d..%d", 8 * g, 8 * g + 7);
-  }
+  // word w of a tile holds unit a2_copy_unit(L) of row 8q + L/8, w = 64 q + L (q = 0, 1)
+  int unit_at[128], row_at[128];
+  std::vector<int> seen(128, 0);
+  for (int q = 0; q < 2; ++q)
+    for (int L = 0; L < 64; ++L) {
+      const int u = sfg::a2_copy_unit(L);
+      CHECK(u >= 0 && u < 8, "unit");
+      unit_at[64 * q + L] = u;
+      row_at[64 * q + L] = 8 * q + (L >> 3);
+      ++seen[row_at[64 * q + L] * 8 + u];
+    }
+  for (int i = 0; i < 128; ++i) CHECK(seen[i] == 1, "(row, unit) %d stored %d times", i, seen[i]);
+  for (int k = 0; k < 2; ++k)
+    for (int g = 0; g < 8; ++g) {
+      int mask = 0;
+      for (int l = 8 * g; l < 8 * g + 8; ++l) {
+        const int w = sfg::a2_read_word(l, k);
+        CHECK(w >= 0 && w < 128, "read word");
+        CHECK(row_at[w] == (l & 15) && unit_at[w] == 4 * k + (l >> 4), "lane %d reads the wrong unit", l);
+        mask |= 1 << (w & 7);
+      }
+      CHECK(mask == 0xff, "bank groups of lanes %d..%d", 8 * g, 8 * g + 7);
+    }
 }
 
 static void check_gemm_columns() {
@@ -428,6 +433,218 @@ static void check_gemm_columns() {
   check_columns<1, false>(1024, 896);     // lm_head-style 128-column tiles
   check_a_tiles();
   printf("gemm columns and weight fragments: ok\n");
+}
+
+// ---------------------------------------------------------------------------
+// Tile GEMM
+// ---------------------------------------------------------------------------
+// One wave of tile_items replayed over an item of nst stages: its copies in issue order
+// (the prologue's, then a window's between the MFMAs), the in-flight counts of its
+// barriers and the order of its LDS reads.  A slot is read only when its copies have
+// landed at the wave's last barrier and filled only when the reads of what it held were
+// done at the barrier that opened the window; a fragment is used only when its read
+// must have landed; every stage and chunk is copied once.
+template <int NMT, int NT>
+static void replay_tile(int w, int nst) {
+  using Sh = sfg::TileShape<NMT, NT>;
+  using St = sfg::TileSteps<NMT, NT>;
+  constexpr int RA = Sh::kRA, RW = Sh::kRW, D = St::kD, CW = Sh::kCW;
+  const int nch = 2 * nst;
+  struct Slot {
+    int held = -1;       // stage or chunk
+    int pending = 0;     // copies not issued yet
+    long long seq = -1;  // the last copy's place in the issue order
+    int read_at = -1;    // last use of a read of it, in barriers passed
+  };
+  std::vector<Slot> a(RA), b(RW);
+  std::vector<int> a_n(nst, 0), b_n(nch, 0);
+  long long issued = 0, landed = 0;   // copies [0, landed) have landed for all waves
+  int barriers = 0;
+  auto copy = [&](Slot& s, int what, int per, std::vector<int>& n) {
+    if (n[what]++ == 0) {
+      CHECK(s.held < 0 || s.read_at < barriers, "slot filled while read");
+      CHECK(s.pending == 0, "slot filled while being filled");
+      s.held = what;
+      s.pending = per;
+    }
+    CHECK(s.held == what, "another fill of the slot");
+    --s.pending;
+    s.seq = issued++;
+  };
+  auto copy_a = [&](int q) { copy(a[q % RA], q, NMT, a_n); };
+  auto copy_w = [&](int c) { copy(b[c % RW], c, w, b_n); };
+  auto barrier = [&](int in_flight) {
+    CHECK(in_flight >= 0 && in_flight < 64, "in flight %d", in_flight);
+    if (issued - in_flight > landed) landed = issued - in_flight;
+    ++barriers;
+  };
+  auto readable = [&](Slot& s, int what) {
+    CHECK(s.held == what && s.pending == 0 && s.seq < landed,
+          "NMT %d NT %d stages %d: %d read before it landed", NMT, NT, nst, what);
+  };
+  // LDS reads: place of the last read into a register, and the stage / chunk it is of
+  long long reads = 0;
+  long long fw_seq[NT], fa_seq[2][NMT];
+  int fw_of[NT], fa_of[2][NMT];
+  auto read_w = [&](int t, int c) {
+    if (c < nch && w) readable(b[c % RW], c);   // (w = 0: other waves bring the weights)
+    fw_seq[t] = reads++;
+    fw_of[t] = c;
+  };
+  auto read_a = [&](int i, int c) {
+    if (c < nch) readable(a[c / 2 % RA], c / 2);
+    fa_seq[c & 1][i] = reads++;
+    fa_of[c & 1][i] = c;
+  };
+  auto open_reads = [&](int j, int c) {
+    if (j == 0)
+      for (int i = 0; i < St::kNA0; ++i) read_a(i, c);
+    if (j == 1)
+      for (int i = St::kNA0; i < NMT; ++i) read_a(i, c);
+    read_w(j, c);
+  };
+  auto use = [&](long long seq, int later) {
+    CHECK(later >= 0 && later <= 15, "lgkmcnt %d", later);
+    CHECK(reads - 1 - seq >= later, "NMT %d NT %d: fragment used before it landed", NMT, NT);
+  };
+  const int first = 1 - 2 * RA < 1 - RW ? 1 - 2 * RA : 1 - RW;
+  for (int v = first; v < 0; ++v) {
+    const int q = (v - 1) / 2 + RA;
+    if ((v & 1) && q >= 0 && q < nst)
+      for (int j = 0; j < NMT; ++j) copy_a(q);
+    if (v - 1 + RW >= 0 && v - 1 + RW < nch)
+      for (int j = 0; j < w; ++j) copy_w(v - 1 + RW);
+  }
+  barrier(nch >= Sh::kTail ? Sh::in_flight_first(w) : 0);
+  for (int j = 0; j < D; ++j) open_reads(j, 0);
+  int fill_a = -1, fill_w = -1;   // stage and chunk the window copies, if any
+  for (int c = 0; c < nch; ++c) {
+    const int k = c & 1;
+    for (int t = 0; t < NT; ++t) {
+      if (t < NT - D) {
+        read_w(t + D, c);
+      } else {
+        if (t == NT - D) {
+          barrier(c + Sh::kTail <= nch ? Sh::in_flight(k, w) : 0);
+          fill_w = c - 1 + RW < nch ? c - 1 + RW : -1;
+          if (k == 1) fill_a = (c - 1) / 2 + RA < nst ? (c - 1) / 2 + RA : -1;
+        }
+        open_reads(t - (NT - D), c + 1);
+      }
+      use(fw_seq[t], St::later(t));
+      CHECK(fw_of[t] == c, "weight fragment of another chunk");
+      b[c % RW].read_at = barriers;
+      if (t == 0)
+        for (int i = 0; i < NMT; ++i) {
+          use(fa_seq[k][i], St::later(t));
+          CHECK(fa_of[k][i] == c, "A fragment of another chunk");
+          a[c / 2 % RA].read_at = barriers;
+        }
+      const bool odd = t >= NT - D ? k == 1 : k == 0;
+      const int n = CW + (odd ? NMT : 0);
+      for (int i = 0; i < n; ++i)
+        if ((NT - D + i * NT / n) % NT == t) {
+          if (odd && i < NMT) {
+            if (fill_a >= 0) copy_a(fill_a);
+          } else if (fill_w >= 0 && i - (odd ? NMT : 0) < w) {
+            copy_w(fill_w);
+          }
+        }
+    }
+  }
+  for (int n : a_n) CHECK(n == NMT, "stage copied %d times", n);
+  for (int n : b_n) CHECK(n == w, "chunk copied %d times", n);
+}
+
+template <int NMT, int NT>
+static void check_tile_shape() {
+  using Sh = sfg::TileShape<NMT, NT>;
+  CHECK(Sh::kWords * 16 <= sfg::kLdsBudget, "ring of NMT %d NT %d", NMT, NT);
+  // a stage's copies: rows 8b .. +8 to words 64 b of the A tiles; a chunk's: a weight
+  // block each; the waves read back whole tiles
+  std::vector<int> aw(Sh::kAW, 0), ww(Sh::kWW, 0);
+  for (int wv = 0; wv < 8; ++wv) {
+    for (int j = 0; j < NMT; ++j)
+      for (int L = 0; L < 64; ++L) {
+        CHECK((wv + 8 * j) * 8 + (L >> 3) < Sh::kRB, "A row");
+        ++aw[wv * 64 + j * 512 + L];
+      }
+    for (int j = 0; j < Sh::kCW; ++j)
+      if (j < Sh::kCW - 1 || Sh::kRem == 0 || wv < Sh::kRem)
+        for (int L = 0; L < 64; ++L) ++ww[wv * 64 + j * 512 + L];
+    const int rgrp = wv & 3, cg = wv >> 2;
+    for (int L = 0; L < 64; ++L) {
+      for (int k = 0; k < 2; ++k)
+        CHECK(rgrp * NMT * 128 + sfg::a2_read_word(L, k) + (NMT - 1) * 128 < Sh::kAW, "A read");
+      CHECK((cg * NT + NT - 1) * 64 + L < Sh::kWW, "weight read");
+    }
+  }
+  for (int n : aw) CHECK(n == 1, "A word copied %d times", n);
+  for (int n : ww) CHECK(n == 1, "weight word copied %d times", n);
+  for (int nst = 1; nst <= 24; ++nst) {
+    replay_tile<NMT, NT>(Sh::kCW, nst);
+    if (Sh::kRem) replay_tile<NMT, NT>(Sh::kCW - 1, nst);
+  }
+}
+
+static void check_tile_gemm() {
+  check_tile_shape<3, 2>();
+  check_tile_shape<3, 3>();
+  check_tile_shape<3, 4>();
+  check_tile_shape<3, 5>();
+  check_tile_shape<3, 6>();
+  check_tile_shape<3, 7>();
+  check_tile_shape<3, 8>();
+  check_tile_shape<4, 2>();
+  check_tile_shape<4, 3>();
+  check_tile_shape<4, 4>();
+  check_tile_shape<4, 5>();
+  check_tile_shape<4, 6>();
+  check_tile_shape<4, 7>();
+  check_tile_shape<4, 8>();
+  // the row blocks cover the rows, the last one not empty
+  for (int M = 1; M <= 256 * sfg::kTileMaxBlocks; ++M) {
+    const int rb = 64 * sfg::tile_nmt(M), nb = (M + rb - 1) / rb;
+    CHECK(nb == sfg::tile_blocks(M), "%d rows: %d blocks of %d", M, nb, rb);
+  }
+  // plans: a tile width that the kernels have, the streaming core's K ranges (so its
+  // sums), and its range slots inside the workspace
+  long long plans = 0;
+  for (int D = 128; D <= 8192; D += 128)
+    for (int K : {64, 128, 192, 896, 1408, 1536, 3584, 4864, 5120, 8960, 14336, 18944, 40960}) {
+      const int T = D / 128, S = K / 64;
+      const sfg::Plan down = sfg::make_plan_split(T, S), qkv = sfg::make_plan_split(T, S, 2);
+      for (int is_qkv = 0; is_qkv < 2; ++is_qkv) {
+        const sfg::Plan& p = is_qkv ? qkv : down;
+        const sfg::TilePlans tp = sfg::make_tile_plans(D / 16, K, false, p.KS);
+        CHECK(tp.ks == p.KS, "ranges");
+        for (int j = 0; j <= p.KS; ++j)
+          CHECK((int)((long long)S * j / tp.ks) == sfg::split_begin(j, p), "range %d", j);
+        for (int M = 1; M <= 1024; M += M < 130 ? 1 : 31) {
+          const int nt = sfg::tile_nt(M, tp), b = sfg::tile_blocks(M);
+          CHECK(nt == 0 || nt == 2 || nt == 4 || nt == 8, "tile width %d", nt);
+          CHECK(sfg::tile_takes(M, tp) == (M > 128 && nt), "takes %d rows", M);
+          const int least = b == 1 ? 3 : b <= 3 ? 2 : 1;
+          CHECK((nt != 0) == (p.KS == 1 || S >= least * p.KS), "rule at %d x %d, %d rows", D, K, M);
+        }
+        const int M = 1024;   // the last range's last element
+        const size_t end = ((size_t)(p.KS - 1) * M + M - 1) * D + D;
+        CHECK(end * sizeof(float) <= (is_qkv ? f_qkv_ws(M, K, D) : f_gemm_ws(M, D, K)),
+              "partial sums of %d x %d", D, K);
+        ++plans;
+      }
+      // o_proj's ranges always suit the tile GEMM
+      const int ks = sfg::rows_splits<1>(1024, D, K, 16);
+      for (int b = 1; b <= 4; ++b)
+        CHECK(sfg::tile_nt(256 * b, sfg::make_tile_plans(D / 16, K, false, ks)) != 0, "o_proj");
+      // gate/up: K as columns
+      const sfg::TilePlans gu = sfg::make_tile_plans(K / 16, D, true, 1);
+      for (int b = 1; b <= 4; ++b) {
+        const int nt = sfg::tile_nt(256 * b, gu);
+        CHECK(nt >= 3 && nt <= 8, "gate/up width %d", nt);
+      }
+    }
+  printf("tile gemm: %lld plans, the ring and read order of 14 shapes\n", plans);
 }
 
 // ---------------------------------------------------------------------------
@@ -700,6 +917,7 @@ int main(int argc, char** argv) {
   check_plans();
   check_rows_plans();
   check_gemm_columns();
+  check_tile_gemm();
   check_lds_paths();
   check_page_addressing();
   check_attention_grid();

@@ -2,7 +2,9 @@
 CPU: tests/cpp/index_check.cpp is compiled with the host C++ compiler against the
 same header the HIP kernels include and run against the built library (for its
 workspace-size queries).  It walks the stream-K GEMM plans, the GEMM output
-columns and packed-weight fragments, the prefix attention's staged-chunk LDS
+columns and packed-weight fragments, the A rows' LDS tiles, the tile GEMM's ring
+(copies, waits and read order replayed per tile shape), row blocks and plans, the
+prefix attention's staged-chunk LDS
 layout with its K and transposed V^T operand reads (emulated element by element,
 with the bank-conflict properties of the swizzles), page-group addressing,
 persistent-grid item walk, chunk ranges and partial slots over the shapes the entry points accept (see the checker's header
@@ -38,8 +40,8 @@ def test_index_maps(checker):
     r = subprocess.run([str(checker), str(lib)], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
     out = r.stdout
-    for family in ("gemm plans", "all-rows GEMM", "gemm columns", "operand reads", "page-group",
-                   "attention grids"):
+    for family in ("gemm plans", "all-rows GEMM", "gemm columns", "tile gemm", "operand reads",
+                   "page-group", "attention grids"):
         assert family in out, out
     assert out.strip().splitlines()[-1].startswith("OK"), out
 
