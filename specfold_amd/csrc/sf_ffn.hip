@@ -380,11 +380,11 @@ Plan gate_up_plan(int I, int S) {
 // The tile GEMM's shapes for a plan whose K ranges are the same for every column (the
 // spread plan's whole K, a split plan's ranges); none for a stream-K plan, whose cuts
 // differ from tile to tile.
-TilePlans down_tiles(const Plan& p, int N, int K) {
-  return p.KS ? make_tile_plans(N / 16, K, false, p.KS) : TilePlans{};
+TilePlans down_tiles(const Plan& p, int N, int K, int rows) {
+  return p.KS && tile_reach(rows, K) ? make_tile_plans(N / 16, K, false, p.KS) : TilePlans{};
 }
-TilePlans gate_up_tiles(const Plan& p, int I, int K) {
-  return p.NU ? make_tile_plans(I / 16, K, true, 1) : TilePlans{};
+TilePlans gate_up_tiles(const Plan& p, int I, int K, int rows) {
+  return p.NU && tile_reach(rows, K) ? make_tile_plans(I / 16, K, true, 1) : TilePlans{};
 }
 
 }  // namespace
@@ -446,7 +446,7 @@ int o_proj_launch(const uint16_t* o_bf, const uint16_t* x, const uint16_t* wo, i
                   uint16_t* zn, void* workspace, hipStream_t st) {
   float* part = reinterpret_cast<float*>(workspace);
   const int ks = rows_splits<1>(M, N, K, kOprojMaxSplits);
-  if (M > 256)
+  if (M > 256 && tile_reach(M, K))
     hipLaunchKernelGGL(o_proj_tile_kernel, dim3(SFG_GRID), dim3(kThreads), 0, st, o_bf, M, wo, K, N,
                        make_tile_plans(N / 16, K, false, ks), part);
   else
@@ -548,7 +548,8 @@ extern "C" int sf_ffn_gate_up(const uint16_t* zn, const int32_t* count, int buck
   ep.out = act;
   ep.ldo = I;
   // whole tiles get SiLU*mul straight from registers, shared tiles in the fix-up
-  launch_sk<2, kSilu>(p, gate_up_tiles(p, I, D), zn, nullptr, D, count, 0, bucket, wg, wu, D, I, part, ep, st);
+  launch_sk<2, kSilu>(p, gate_up_tiles(p, I, D, bucket), zn, nullptr, D, count, 0, bucket, wg, wu, D,
+                      I, part, ep, st);
   if (p.U < p.S)
     hipLaunchKernelGGL(silu_fixup_kernel, dim3(p.T, (bucket + kFixRows - 1) / kFixRows), dim3(256),
                        0, st, part, p, bucket, count, I, act);
@@ -569,7 +570,7 @@ extern "C" int sf_ffn_down_scatter(const uint16_t* act, const int32_t* count, in
   ep.rows = rows;
   ep.out = ffn;
   ep.ldo = D;
-  const TilePlans tp = down_tiles(p, D, I);
+  const TilePlans tp = down_tiles(p, D, I, bucket);
   launch_sk<1, kScatter>(p, tp, act, nullptr, I, count, 0, bucket, wd, nullptr, I, D, part, ep, st);
   hipLaunchKernelGGL(down_fixup_kernel, dim3(p.T, (bucket + kFixRows - 1) / kFixRows), dim3(256), 0,
                      st, part, p, bucket, rows, count, D, ffn, tp);

@@ -112,7 +112,7 @@ SF_DEV void tile_items(const TileGemm& g, int M, int n_ranges, sf_u32x4* ring, c
 
     // this wave's copies.  A block b = wv + 8j of a stage: rows 8b .. +8 (rows past the
     // end repeat the last); weight block w = wv + 8j of a chunk: tile w.  A uniform
-    // base advancing per stage / chunk plus this lane's 32-bit offset.
+    // base advancing per stage / chunk plus this lane's 32-bit offset (tile_reach).
     const char* abase = reinterpret_cast<const char*>(g.A) + (size_t)sa * 128;
     uint32_t aoff[NMT];
 #pragma unroll

@@ -388,7 +388,7 @@ extern "C" int sf_head_logits_rows(const uint16_t* x, int M, const uint16_t* w, 
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (Mo <= HeadMain128::kRows)
     head_launch<HeadMain128, HeadTail128>(x, Mo, hr, w, D, V, logits, ld_out, st);
-  else if (head_tiles(Mo, D))
+  else if (head_tiles(Mo, D) && tile_reach(M, D))
     head_tile_launch(x, Mo, hr, w, D, V, logits, ld_out, st);
   else
     head_launch<HeadMain, HeadTail>(x, Mo, hr, w, D, V, logits, ld_out, st);

@@ -337,6 +337,9 @@ struct TilePlans {
   unsigned nt = 0;   // byte tile_blocks(M) - 1: NT, or 0: such rows stay on the streaming core
 };
 SF_IDX int tile_nt(int M, const TilePlans& p) { return (p.nt >> (8 * (tile_blocks(M) - 1))) & 255; }
+// A table of `rows` rows of K that the tile GEMM's 32-bit row offsets reach (64-bit ones
+// take its copies a few cycles more: a prefill of 2048 tokens 6812 -> 6867 us).
+inline bool tile_reach(long long rows, int K) { return rows * K * 2 <= 1ll << 32; }
 // Whether the tile GEMM computes M rows.
 SF_IDX bool tile_takes(int M, const TilePlans& p) { return M > kTileRows && tile_nt(M, p) != 0; }
 // Cycles of a workgroup per 32-wide K chunk: the LDS operand reads of 8 waves

@@ -89,8 +89,8 @@ Plan qkv_plan(int n_qkv, int D) {
   const int T = n_qkv / 128, S = D / kKC;
   return T < SFG_GRID ? make_plan_split(T, S, 2) : make_plan(T, S);
 }
-TilePlans qkv_tiles(const Plan& p, int n_qkv, int D) {
-  return p.KS ? make_tile_plans(n_qkv / 16, D, false, p.KS) : TilePlans{};
+TilePlans qkv_tiles(const Plan& p, int n_qkv, int D, int rows) {
+  return p.KS && tile_reach(rows, D) ? make_tile_plans(n_qkv / 16, D, false, p.KS) : TilePlans{};
 }
 
 }  // namespace
@@ -120,7 +120,7 @@ extern "C" int sf_qkv_rope(const uint16_t* xn, const int32_t* rows, const int32_
   if (workspace_bytes < sf_qkv_workspace_bytes(bucket, D, n_qkv)) return SF_ERR_WORKSPACE;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const Plan p = qkv_plan(n_qkv, D);
-  const TilePlans tp = qkv_tiles(p, n_qkv, D);
+  const TilePlans tp = qkv_tiles(p, n_qkv, D, BN);
   float* part = reinterpret_cast<float*>(workspace);
   launch_sk<1, kPart>(p, tp, xn, rows, D, count, 0, bucket, w_qkv, nullptr, D, n_qkv, part, Epi{}, st);
   dim3 g2(min(bucket, 128), (H + 2 * Hkv + 3) / 4);
@@ -155,7 +155,7 @@ extern "C" int sf_qkv_rope_branches(const uint16_t* xn, const int32_t* rows,
   if (workspace_bytes < sf_qkv_workspace_bytes(bucket, D, n_qkv)) return SF_ERR_WORKSPACE;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const Plan p = qkv_plan(n_qkv, D);
-  const TilePlans tp = qkv_tiles(p, n_qkv, D);
+  const TilePlans tp = qkv_tiles(p, n_qkv, D, BN);
   float* part = reinterpret_cast<float*>(workspace);
   launch_sk<1, kPart>(p, tp, xn, rows, D, count, 0, bucket, w_qkv, nullptr, D, n_qkv, part, Epi{}, st);
   dim3 g2(min(bucket, 128), (H + 2 * Hkv + 3) / 4);
@@ -194,7 +194,7 @@ extern "C" int sf_qkv_rope_gated(const uint16_t* xn, const int8_t* rec, const in
   if (workspace_bytes < sf_qkv_workspace_bytes(bucket, D, n_qkv)) return SF_ERR_WORKSPACE;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const Plan p = qkv_plan(n_qkv, D);
-  const TilePlans tp = qkv_tiles(p, n_qkv, D);
+  const TilePlans tp = qkv_tiles(p, n_qkv, D, B1 * N);
   float* part = reinterpret_cast<float*>(workspace);
   const GateIn gate{rec, par, B1, N, GateOut{f, src, rows, count, seg, segcnt, slot}};
   launch_sk<1, kPart, true>(p, tp, xn, nullptr, D, nullptr, 0, bucket, w_qkv, nullptr, D, n_qkv, part,
