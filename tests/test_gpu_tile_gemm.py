@@ -2,7 +2,8 @@
 of its row blocks (64·NMT rows, blocks of at most 256), column tiles and K ranges:
 against float64 products with the other GEMM tests' bound, and bit for bit against
 the streaming core's results for the same rows (a row's sums do not depend on how
-many rows are computed with it)."""
+many rows are computed with it).  Short K ranges stay on the streaming core at some of
+these row counts (make_tile_plans): both sides of that rule are among the shapes."""
 
 import pytest
 import torch
@@ -74,3 +75,56 @@ def test_qkv_rows(M, D, H, Hkv):
     assert torch.equal(out[:100], few[:100])
     assert torch.all(out[M:] == 3.0)
     close_bf16(out[:M], mm64(x[:M], w), atol=acc_bound(x[:M], w))
+
+
+# 144 recomputed rows of 640 (one row block) and 300 of 1024 (two), scattered; 48 column
+# tiles in 5 ranges of 6 stages
+@pytest.mark.parametrize("count,BN", [(144, 640), (300, 1024)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_qkv_gathered_rows(count, BN, gated):
+    """The rows of a verify step of several sequences: gathered from among more flat
+    rows, through sf_qkv_rope's row list and sf_qkv_rope_gated's compaction of rec."""
+    D, H, Hkv, N = 2048, 32, 8, 32
+    g = torch.Generator().manual_seed(count)
+    nq = (H + 2 * Hkv) * 128
+    x, w = rnd(BN, D, gen=g), rnd(nq, D, std=0.05, gen=g)
+    wp = packed(w)
+    pick = torch.randperm(BN, generator=g)[:count].sort().values
+    cos = torch.ones(N, 128, dtype=torch.bfloat16, device="cuda")   # no rotation
+    sin = torch.zeros_like(cos)
+    ws = zeros_ws(_lib.qkv_workspace_bytes(BN, D, nq))
+
+    def outputs():
+        return (torch.full((BN + 1, H * 128), 3.0, dtype=torch.bfloat16, device="cuda"),
+                torch.full((BN + 1, 2 * Hkv * 128), 3.0, dtype=torch.bfloat16, device="cuda"))
+
+    def run(pick):
+        q, kv = outputs()
+        rows = torch.full((BN,), BN, dtype=torch.int32)
+        rows[:len(pick)] = pick
+        _lib.qkv_rope(x, rows.cuda(), torch.tensor([len(pick)], dtype=torch.int32).cuda(), BN, BN, wp,
+                      None, cos, sin, None, N, D, H, Hkv, 128, q, kv, ws)
+        return torch.cat([q, kv], dim=1)
+
+    if gated:
+        q, kv = outputs()
+        rec = torch.zeros(BN, dtype=torch.int8)
+        rec[pick] = 1
+        f, src, rows, seg, slot = (torch.zeros(BN, dtype=torch.int32, device="cuda") for _ in range(5))
+        cnt = torch.zeros(1, dtype=torch.int32, device="cuda")
+        segcnt = torch.zeros(BN // N, dtype=torch.int32, device="cuda")
+        par = torch.arange(BN // N, dtype=torch.int32, device="cuda")   # every branch a root
+        _lib.qkv_rope_gated(x, rec.cuda(), par, BN // N, N, BN, f, src, rows, cnt, seg, segcnt, slot,
+                            wp, None, cos, sin, None, D, H, Hkv, 128, q, kv, ws)
+        assert int(cnt) == count and torch.equal(rows[:count].cpu().long(), pick)
+        out = torch.cat([q, kv], dim=1)
+    else:
+        out = run(pick)
+    parts = [run(pick[i:i + 100]) for i in range(0, count, 100)]
+    torch.cuda.synchronize()
+    others = torch.ones(BN + 1, dtype=torch.bool)
+    others[pick] = False
+    assert torch.all(out[others] == 3.0)
+    for i, few in zip(range(0, count, 100), parts):
+        assert torch.equal(out[pick[i:i + 100]], few[pick[i:i + 100]])
+    close_bf16(out[pick], mm64(x[pick], w), atol=acc_bound(x[pick], w))
