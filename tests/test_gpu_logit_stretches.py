@@ -1,12 +1,14 @@
 """The greedy statistics at the edges of the stretches kept in LDS: rows of few, exactly
-the most, one more and very many distinct 64-key stretches give the same numbers as the
-float64 softmax and leave the histogram zero for the next call (each row is followed by
-a plain one through the same workspace)."""
+the most, one more and very many distinct 64-key stretches give the numbers of the
+float64 softmax, the nucleus cut of the reference's rule (by the walk in LDS and the one
+in memory) and its greedy token, and leave the histogram zero for the next call (each
+row is followed by a plain one through the same workspace)."""
 
 import pytest
 import torch
 
 from specfold_amd import _lib
+from tests.test_gpu_logit_stats import nucleus_mass64
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +47,15 @@ def test_stretches(stretches):
         assert torch.equal(st.top_val.double(), -order.values[:, :8])
         assert torch.equal(st.znuc, got[0].znuc) and torch.equal(st.greedy_tok, got[0].greedy_tok)
     assert torch.all(got[0].znuc <= got[0].zfull * (1 + 1e-6))
+    for top_p in (0.3, 0.8, 0.95, 0.999):
+        st = _lib.logit_stats(x, top_p)
+        zn, _ = nucleus_mass64(x, top_p)
+        # the cut moves by one token (e <= 1) where the bf16 sum rounds across top_p
+        assert torch.all((st.znuc.double() - zn).abs() <= 1e-4 * z + 1.0), (top_p, st.znuc, zn)
+        # the kernel's own nucleus mass, fp32: its bf16 reciprocal, and the lowest index
+        # whose bf16 probability is as large (torch's bf16 softmax of the kept logits is up
+        # to two bf16 steps off at a flat row's mass, so it is no oracle here)
+        assert torch.equal(st.conf, (1 / st.znuc).to(torch.bfloat16).float())
+        e = (d - d.amax(-1, keepdim=True)).exp()
+        prob = (e / st.znuc.double()[:, None]).float().to(torch.bfloat16)
+        assert torch.equal(st.greedy_tok.long(), (prob == prob.amax(-1, keepdim=True)).int().argmax(-1))
