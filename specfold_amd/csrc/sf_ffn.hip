@@ -379,7 +379,9 @@ Plan gate_up_plan(int I, int S) {
 
 // The tile GEMM's shapes for a plan whose K ranges are the same for every column (the
 // spread plan's whole K, a split plan's ranges); none for a stream-K plan, whose cuts
-// differ from tile to tile.
+// differ from tile to tile: gate/up of I < 8192 or I > 32768 takes more than 128 rows in
+// passes of 128 (256 / 1024 rows at 2048 x 5632 53 / 190 us; at 2048 x 8192 32 / 64 on
+// the tile GEMM, where passes took 55 / 207).
 TilePlans down_tiles(const Plan& p, int N, int K, int rows) {
   return p.KS && tile_reach(rows, K) ? make_tile_plans(N / 16, K, false, p.KS) : TilePlans{};
 }
@@ -548,8 +550,8 @@ extern "C" int sf_ffn_gate_up(const uint16_t* zn, const int32_t* count, int buck
   ep.out = act;
   ep.ldo = I;
   // whole tiles get SiLU*mul straight from registers, shared tiles in the fix-up
-  launch_sk<2, kSilu>(p, gate_up_tiles(p, I, D, bucket), zn, nullptr, D, count, 0, bucket, wg, wu, D,
-                      I, part, ep, st);
+  launch_sk<2, kSilu>(p, gate_up_tiles(p, I, D, bucket), zn, nullptr, D, count, 0, bucket, wg, wu,
+                      D, I, part, ep, st);
   if (p.U < p.S)
     hipLaunchKernelGGL(silu_fixup_kernel, dim3(p.T, (bucket + kFixRows - 1) / kFixRows), dim3(256),
                        0, st, part, p, bucket, count, I, act);

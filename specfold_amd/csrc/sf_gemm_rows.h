@@ -147,8 +147,8 @@ void gemm_rows_kernel(const uint16_t* __restrict__ A, int M, const uint16_t* __r
   }
 }
 
-// One launch per 256 rows: rows [m0, m0 + 256) of A, out and every partial slot
-// (slot stride M·N).  N must be a multiple of 16·WN·4 and of 128·rows_wn(1).
+// One launch per 256 rows (o_proj of more comes here only where the tile GEMM's offsets
+// do not reach): rows [m0, m0 + 256) of A, out and every partial slot (slot stride M·N).  N must be a multiple of 16·WN·4 and of 128·rows_wn(1).
 template <int WN, int MODE>
 inline void launch_rows(const uint16_t* A, int M, const uint16_t* W, int K, int N, int ks_max,
                         float* part, uint16_t* out, hipStream_t st) {

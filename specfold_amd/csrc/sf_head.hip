@@ -264,10 +264,14 @@ void head_kernel(const uint16_t* __restrict__ X, int Mo, int m0, HeadRows hr,
 // above bit for bit (K ascending in one accumulator).  Its cost follows the row blocks
 // (192 or 256 rows each, several in one launch), where the kernel above pays a whole
 // pass over the weights per 256 rows whatever they hold.
-// Stores: non-temporal up to 256 rows (a verify step), plain above (prompts).  32 bytes of
-// a row a store, plain ones leave L2 as whole lines (1024 rows of 152064: 1030 -> 958 us),
-// but the next forward's weight streams find them there: 256 rows on plain tile stores
-// took 287 us against a pass's 296, and the 8-layer verify step 1568 against 1557.
+// Stores: non-temporal for the one-block counts that come here (129 to 192 rows, D >= 2048:
+// verify steps of 5 and 6 branches), plain above 256 rows (prompts, steps of several
+// sequences).  32 bytes of a row a store, plain ones leave L2 as whole lines (1024 rows of
+// 152064: 1030 -> 958 us), but the next forward's weight streams find them there: 256 rows
+// on plain tile stores took 287 us against a pass's 296, and the 8-layer verify step 1568
+// against 1557 (193 to 256 rows stay on the pass).  A step of several sequences is as fast
+// either way (6 layers, non-temporal / plain, us: 4 x 5 branches 2793 / 2787 at 7B widths,
+// 2836 / 2830 at 8B; 2 x 5 1863 / 1855, 1858 / 1861; 4 x 8 3171 / 3174, 3285 / 3286).
 struct HeadTileStore {
   HeadRows hr;
   uint16_t* out;
@@ -324,7 +328,8 @@ bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0;
 namespace {
 
 // Whole rounds of the main shape's tiles (one per CU), the rest in the tail shape's
-// (the partial last round spread over up to twice the CUs); passes of Main::kRows.
+// (the partial last round spread over up to twice the CUs); passes of Main::kRows (one,
+// but for rows that the tile GEMM's offsets do not reach).
 template <class Main, class Tail>
 void head_launch(const uint16_t* x, int Mo, const HeadRows& hr, const uint16_t* w, int D, int V,
                  uint16_t* logits, long long ld_out, hipStream_t st) {

@@ -238,8 +238,8 @@ template <int WN>
 inline int rows_tiles(int N, int rg) { return N / (16 * rows_wn<WN>(rg) * (8 / rg)); }
 // K stages of an all-rows GEMM (32·CPS each).
 inline int rows_stages(int K) { return K / (32 * SFG_ROWS_CPS); }
-// K ranges of an all-rows GEMM over M rows: the first pass's plan, used by every
-// pass (the consumer adds the same number of partial slots for every row).
+// K ranges of an all-rows GEMM over M rows: those of a pass of up to 256, whatever
+// computes more rows (the consumer adds the same number of partial slots for each).
 template <int WN>
 inline int rows_splits(int M, int N, int K, int ks_max) {
   const int rg = rows_rg(sf_imin(256, M));

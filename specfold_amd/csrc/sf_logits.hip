@@ -94,29 +94,25 @@ SF_DEV uint32_t rank_key(uint32_t b) {
   return bf16_key(a == 0u ? 0u : b);
 }
 
-template <typename K>
-SF_DEV K wave_max(K x) {
+SF_DEV uint32_t wave_max(uint32_t x) {
 #pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
-    const K y = __shfl_xor(x, o, 64);
-    x = x > y ? x : y;
-  }
+  for (int o = 32; o >= 1; o >>= 1) x = max(x, (uint32_t)__shfl_xor(x, o, 64));
   return x;
 }
 
 // Top-8 of a wave from per-lane lists of L keys in descending order (nonzero keys
 // distinct, 0 = empty): 8 rounds of a wave maximum, the winning lane popping its
 // list's head.  Every lane gets the 8 in `out`, largest first.
-template <int L, typename K>
-SF_DEV void wave_top8(K (&l)[L], K (&out)[kTop]) {
+template <int L>
+SF_DEV void wave_top8(uint32_t (&l)[L], uint32_t (&out)[kTop]) {
 #pragma unroll
   for (int r = 0; r < kTop; ++r) {
-    const K w = wave_max(l[0]);
+    const uint32_t w = wave_max(l[0]);
     out[r] = w;
     const bool pop = l[0] == w;
 #pragma unroll
     for (int k = 0; k + 1 < L; ++k) l[k] = pop ? l[k + 1] : l[k];
-    l[L - 1] = pop ? K(0) : l[L - 1];
+    l[L - 1] = pop ? 0u : l[L - 1];
   }
 }
 
@@ -201,7 +197,7 @@ __global__ __launch_bounds__(kSliceThreads) void sf_logit_slice_kernel(
   // the slice's top-8: each wave's, then wave 0 merges the waves' 8 x 8
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   uint32_t wt[kTop];
-  wave_top8<kTop>(top, wt);
+  wave_top8(top, wt);
   if (lane == 0) {
 #pragma unroll
     for (int r = 0; r < kTop; ++r) s_top[wv * kTop + r] = wt[r];
@@ -210,7 +206,7 @@ __global__ __launch_bounds__(kSliceThreads) void sf_logit_slice_kernel(
   if (wv == 0) {
     uint32_t one[1] = {s_top[lane]};
     uint32_t bt[kTop];
-    wave_top8<1>(one, bt);
+    wave_top8(one, bt);
     if (lane < kTop) {
       uint32_t b = bt[0];
 #pragma unroll

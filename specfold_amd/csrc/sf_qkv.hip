@@ -6,9 +6,9 @@
 // bf16 op rounded) and the Triton kernel specfold/generate/triton_kernels.py:29-87.
 //
 // GEMM: out[m, c] = sum_k xn[rows[m], k] * w[c, k]; M = count <= bucket,
-// N = (H + 2*Hkv)*hd, K = D, on the stream-K weight-streaming core of
-// sf_gemm_core.h with one head (128 columns) per tile, every piece to fp32
-// partial slots; the epilogue kernel sums a head's slots in slot order
+// N = (H + 2*Hkv)*hd, K = D, on the weight-streaming core of sf_gemm_core.h with
+// one head (128 columns) per tile, each tile cut into whole K ranges (qkv_plan), every
+// range to fp32 partial slots; the epilogue kernel sums a head's slots in slot order
 // (deterministic), adds the bias, rounds, ropes and scatters.
 #include "sf_gemm_core.h"
 
@@ -84,7 +84,12 @@ __global__ __launch_bounds__(256) void sf_qkv_epilogue_kernel(
 // are fewer than the grid: the same ranges for every head, so that the tile GEMM (more
 // than 128 rows) gives every row the streaming core's sums.  A range holds at least
 // two 64-K stages: shorter ones are all ring fill, and their partial slots cost the
-// epilogue more than the idle CUs do the GEMM.
+// epilogue more than the idle CUs do the GEMM.  Against stream-K over the full grid, us
+// (GEMM and epilogue; one workgroup per range, so none straddles two heads and fills its
+// ring twice): 32 / 64 / 128 rows at 4096 x 6144 (240 workgroups of 12-13 stages) 20.1 /
+// 23.3 / 29.1 -> 19.1 / 19.3 / 21.3, at 5120 x 7168 (224 of 20) 24.1 / 27.8 / 33.8 -> 22.2
+// / 24.4 / 29.2; at 3584 x 4608 the ranges are the same, at 1536 x 2048 a call is as long
+// as its launches (19 us) either way.
 Plan qkv_plan(int n_qkv, int D) {
   const int T = n_qkv / 128, S = D / kKC;
   return T < SFG_GRID ? make_plan_split(T, S, 2) : make_plan(T, S);
@@ -122,7 +127,8 @@ extern "C" int sf_qkv_rope(const uint16_t* xn, const int32_t* rows, const int32_
   const Plan p = qkv_plan(n_qkv, D);
   const TilePlans tp = qkv_tiles(p, n_qkv, D, BN);
   float* part = reinterpret_cast<float*>(workspace);
-  launch_sk<1, kPart>(p, tp, xn, rows, D, count, 0, bucket, w_qkv, nullptr, D, n_qkv, part, Epi{}, st);
+  launch_sk<1, kPart>(p, tp, xn, rows, D, count, 0, bucket, w_qkv, nullptr, D, n_qkv, part, Epi{},
+                      st);
   dim3 g2(min(bucket, 128), (H + 2 * Hkv + 3) / 4);
   hipLaunchKernelGGL(sf_qkv_epilogue_kernel<false>, g2, dim3(256), 0, st, part, p, bucket, n_qkv, rows,
                      count, b_qkv, cos_tab, sin_tab, pos0, table_rows, q_scale, N, H, Hkv, q_buf,
@@ -157,7 +163,8 @@ extern "C" int sf_qkv_rope_branches(const uint16_t* xn, const int32_t* rows,
   const Plan p = qkv_plan(n_qkv, D);
   const TilePlans tp = qkv_tiles(p, n_qkv, D, BN);
   float* part = reinterpret_cast<float*>(workspace);
-  launch_sk<1, kPart>(p, tp, xn, rows, D, count, 0, bucket, w_qkv, nullptr, D, n_qkv, part, Epi{}, st);
+  launch_sk<1, kPart>(p, tp, xn, rows, D, count, 0, bucket, w_qkv, nullptr, D, n_qkv, part, Epi{},
+                      st);
   dim3 g2(min(bucket, 128), (H + 2 * Hkv + 3) / 4);
   hipLaunchKernelGGL(sf_qkv_epilogue_kernel<true>, g2, dim3(256), 0, st, part, p, bucket, n_qkv,
                      rows, count, b_qkv, cos_tab, sin_tab, pos0_branch, table_rows, q_scale_rows,
@@ -197,8 +204,8 @@ extern "C" int sf_qkv_rope_gated(const uint16_t* xn, const int8_t* rec, const in
   const TilePlans tp = qkv_tiles(p, n_qkv, D, B1 * N);
   float* part = reinterpret_cast<float*>(workspace);
   const GateIn gate{rec, par, B1, N, GateOut{f, src, rows, count, seg, segcnt, slot}};
-  launch_sk<1, kPart, true>(p, tp, xn, nullptr, D, nullptr, 0, bucket, w_qkv, nullptr, D, n_qkv, part,
-                            Epi{}, st, gate);
+  launch_sk<1, kPart, true>(p, tp, xn, nullptr, D, nullptr, 0, bucket, w_qkv, nullptr, D, n_qkv,
+                            part, Epi{}, st, gate);
   dim3 g2(min(bucket, 128), (H + 2 * Hkv + 3) / 4);
   if (pos0_per_branch)
     hipLaunchKernelGGL(sf_qkv_epilogue_kernel<true>, g2, dim3(256), 0, st, part, p, bucket, n_qkv,
