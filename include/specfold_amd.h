@@ -255,7 +255,8 @@ int sf_attn_rows(const uint16_t* q_buf, const uint16_t* kv_buf, const uint16_t* 
  * specfold/generate/fastdllm_v2_generation.py:510-524 (bidirectional in a block, causal
  * across blocks); block = 1: causal (specfold/generate/nld_generation.py:186-194).
  * Writes o_bf for rows 0 .. n - 1 (row stride H*hd).  Same softmax arithmetic as
- * sf_attn_prefix_block.  workspace: sf_attn_chunk_workspace_bytes(n, H), 16-byte aligned.
+ * sf_attn_prefix_block; keys and values that a row does not see never reach it, NaN and
+ * inf among them.  workspace: sf_attn_chunk_workspace_bytes(n, H), 16-byte aligned.
  * Limits: hd == 128, H % Hkv == 0, H/Hkv <= 8, 1 <= n <= 1024, n <= P <= 32768, the page
  * sizes of sf_attn_prefix_block.  No counterpart in the reference, whose prefill is
  * inside the checkpoint's remote code.

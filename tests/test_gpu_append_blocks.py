@@ -53,6 +53,38 @@ def test_attn_chunk(n, prefix, block, H, Hkv, shuffled):
     assert torch.all(o[n] == 7.0)
 
 
+@pytest.mark.parametrize("n,prefix,block,H,Hkv,at", [
+    (64, 0, 32, 28, 4, 40), (1000, 77, 1, 32, 8, 600), (1024, 1024, 32, 28, 4, 1500),
+    (200, 5000, 16, 40, 8, 5199), (129, 0, 64, 4, 4, 128)])
+def test_attn_chunk_hidden_value_not_finite(n, prefix, block, H, Hkv, at):
+    """An inf among the values reaches the rows that see its position, in its dims: all
+    else is as over the finite cache (the oracle: zeros in its place)."""
+    g = torch.Generator(device="cuda").manual_seed(n + at)
+    P = prefix + n
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g, device="cuda").to(torch.bfloat16)
+    q, k, v = rnd(n, H, HD), rnd(Hkv, P, HD), rnd(Hkv, P, HD)
+    vz = v.clone()
+    v[0, at, [3, 64]], vz[0, at, [3, 64]] = float("inf"), 0
+    cache = PagedKVCache(1, Hkv, HD, P, page_order="shuffled", seed=3)
+    cache.load_dense([(k[None], v[None])])
+    vw = cache.view(0)
+    o = torch.empty(n, H * HD, dtype=torch.bfloat16, device="cuda")
+    ws = torch.full((_lib.attn_chunk_workspace_bytes(n, H),), 255, dtype=torch.uint8, device="cuda")
+    _lib.attn_chunk(q, vw.k, vw.v, vw.page_table, P, vw.page_size, vw.page_stride, vw.head_stride,
+                    n, block, H, Hkv, HD, HD ** -0.5, o, ws)
+    ref = chunk_attention(q, k, vz, n, block)
+    got = o.double().view(n, H, HD)
+    m = torch.arange(n, device="cuda")
+    sees = at < prefix + ((m // block + 1) * block).clamp(max=n)
+    hit = torch.zeros(n, H, HD, dtype=torch.bool, device="cuda")
+    hit[:, :H // Hkv, [3, 64]] = sees[:, None, None]
+    assert bool(sees.any()) and not torch.any(got[hit].isfinite())
+    d = (got - ref).abs()
+    assert torch.all((d <= 2 ** -8 * ref.abs() + 2 ** -14 * vz.abs().max().double())[~hit])
+
+
 def _executor(family):
     from specfold_amd.generate.fastdllm_model_executor import FastDLLMModelExecutor
     from specfold_amd.generate.nld_model_executor import NLDModelExecutor
@@ -95,6 +127,25 @@ def test_prompt_matches_blocks(family, lengths):
     for li in range(3):
         for a, b in zip(whole[li], parts[li]):
             assert (a.double() - b.double()).norm() / b.double().norm() < 1.6e-2
+
+
+def test_prompt_repeats_itself():
+    """The same prompt twice, another one of other lengths in between through the same
+    buffers: the same bits."""
+    ex = _executor("nld_diffusion")
+    g = torch.Generator().manual_seed(7)
+    t, other = (torch.randint(0, 900, (1, n), generator=g) for n in (1150, 990))
+
+    def run(t):
+        cache = ex.new_cache()
+        return ex.forward(t, cache, use_cache=True, use_causal_mask=True).logits.clone(), cache
+    first, ca = run(t)
+    run(other)
+    again, cb = run(t)
+    assert torch.equal(first, again)
+    for li in range(3):
+        for a, b in zip(ca[li], cb[li]):
+            assert torch.equal(a, b)
 
 
 def test_full_cache_is_refused_as_before():
